@@ -44,7 +44,7 @@ def build_oracle() -> Path:
 
 
 def build_reference() -> list[Path]:
-    if not REF_ROOT.exists():
+    if not (REF_ROOT / "tools/trace/cpu_mxfp4_vnni.cpp").exists():   # also when the folder is there but empty
         print(f"reference sources not present at {REF_ROOT}; skipping oracle/_ref", file=sys.stderr)
         return []
     REF_OUT.mkdir(exist_ok=True)
