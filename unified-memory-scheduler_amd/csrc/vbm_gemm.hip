@@ -57,6 +57,15 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T * cst(const
     return (const __attribute__((address_space(4))) T *)(p);
 }
 
+// A wave-uniform pointer the compiler holds in vector registers, back in scalar ones.
+template <class T>
+__device__ __forceinline__ T * uniform_ptr(T * p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+    return reinterpret_cast<T *>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 struct GemmShape {
     int nb, rows, interleave;
     size_t slot_bytes;
@@ -80,6 +89,7 @@ struct GemmArgs {
     const float * row_scale;   // epilogue 0: per-job factor applied after the bias (routing weights), or null
     float * dst;               // epilogue 0: [job][rows]
     int row_pairs;             // 64-row tile pairs of the bank
+    int row_units;             // MXFP4: 128-row units of the bank
     uint8_t * rows_out;        // epilogue 1: GLU output rows for the down projection (out_lay)
     GemmRowLayout out_lay;
     int activation;
@@ -855,6 +865,452 @@ __global__ __launch_bounds__(kGemmThreads, (TYPE == 8 && !FLAGGED) ? 3 : 1) void
     }
 }
 
+// ------------------------------------------------------------------------ MXFP4 grouped GEMM
+// A wave owns 64 bank rows (a tile pair, so a whole 32-element GLU block of an interleaved bank) and
+// up to 64 jobs: a 4 x 4 grid of 16 x 16 fragments. Its weights go from the bank straight into
+// registers, one 8-block group ahead (no other wave of the workgroup needs them; as A operand, lane
+// (q, r) of a fragment takes the 16-byte entries of slices 2q and 2q + 1 of its row as stored), and
+// only the activation rows, which every wave reads, are staged in LDS. A workgroup (4 waves) takes
+//   - job tiles of at most 64 live jobs: four tile pairs (256 rows) x the tile, so the activation
+//     rows are fetched once per 256 rows;
+//   - larger ones (up to 128): two tile pairs x two halves of the live jobs, split at a multiple of 16.
+// Stages hold four blocks (half a bank group) of every live job's codes and block scales, two of
+// them in turn, so one wait and one barrier per four blocks.
+// Each wave's block products are summed with one FMA per output and block in block order, as in
+// every form of this kernel: the split over waves changes no bit of the result.
+//
+// The block exponents ride in the A operand when every exponent e of the wave's rows lies in
+// [-14, 12] (2^(e+1) times the e2m1 values is then an exact normal f16), which the wave checks
+// first; otherwise, and for waves holding -128 codes (FLAGGED), the wave takes the general path:
+// doubled-integer operands, ldexp(d_act, e) per output, and the exact -128 correction.
+struct MxStageLayout {
+    static constexpr int kJobs = 128, CB = 4;
+    static constexpr int ROW = CB * 64;                        // f16 codes of a job and stage
+    static constexpr int DA = kJobs * CB * 4;                  // [job][4 blocks] fp32 block scales, both stages first
+    static constexpr int OFF_EXP = 2 * DA;                     // [group & 1][wave][64 rows] x 8 exponent bytes
+    static constexpr int OFF_ACT = OFF_EXP + 2 * 4 * 512;      // (last: every LDS read then has a 16-bit offset)
+    static constexpr int ACT = kJobs * ROW;
+    static constexpr int BYTES = OFF_ACT + 2 * ACT;
+};
+// Weights of a wave and group: entry [i][s] is slice 2q + s of row 16i + lr (dword d holds blocks
+// 2d, 2d + 1). Their exponents are staged in LDS: as registers too they would spill.
+struct MxGroupRegs {
+    u32x4g c[4][2];
+};
+constexpr int kMxGroupLoads = 8;   // vector loads of a group
+
+// Every stored exponent byte (signed e) of the dword in [-14, 12]: e + 14 and e + 19 both in [0, 32).
+__device__ __forceinline__ unsigned mx_unfoldable(unsigned w) {
+    const unsigned lo = w & 0x7F7F7F7Fu, sg = w & 0x80808080u;
+    return (((lo + 0x0E0E0E0Eu) ^ sg) | ((lo + 0x13131313u) ^ sg)) & 0xE0E0E0E0u;
+}
+
+template <int EPI, bool FLAGGED>
+__global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs A) {
+    using L = MxStageLayout;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[L::BYTES];
+    // XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of
+    // (tile, row unit) items; the units of one job tile share its activation rows in one L2.
+    const int n_items = *cst<int32_t>(A.n_tiles) * A.row_units;
+    const int per_xcd = (n_items + 7) >> 3;
+    const int slot8 = static_cast<int>(blockIdx.x >> 3);
+    const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
+    if (slot8 >= per_xcd || item >= n_items) return;
+    const int ti = item / A.row_units;
+    const int unit = item - ti * A.row_units;          // 128 rows; 256 for tiles of at most 64 jobs
+    const int expert = cst<int32_t>(A.tile_expert)[ti];
+    const int j0 = cst<int32_t>(A.tile_start)[ti];
+    const int count = cst<int32_t>(A.counts)[expert];
+    const int joff = cst<int32_t>(A.offsets)[expert];
+    const int slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[expert] : expert;
+    const GemmShape S = A.shape;
+    const int live = count - j0 < L::kJobs ? count - j0 : L::kJobs;
+    const bool wide = live <= 64;
+    const int pair0 = unit * (wide ? 4 : 2), n_pairs = wide ? 4 : 2;
+    if (pair0 * 64 >= S.rows) return;
+    if (slot < 0 || slot >= S.n_slots) {
+        // Expert not resident in this bank: NaN outputs, as in the decode kernels (a tile filter
+        // removes the experts a pass skips on purpose, so this is a bad map).
+        const float nan = __builtin_nanf("");
+        if (EPI == 0) {
+            for (int i = threadIdx.x; i < live * n_pairs * 64; i += kGemmThreads) {
+                const int64_t brow = static_cast<int64_t>(pair0) * 64 + i % (n_pairs * 64);
+                if (brow < S.rows)
+                    A.dst[static_cast<size_t>(A.jobs[joff + j0 + i / (n_pairs * 64)]) * S.rows + ggml_row(brow, S.rows, S.interleave)] = nan;
+            }
+        } else {
+            for (int i = threadIdx.x; i < live * n_pairs; i += kGemmThreads)
+                if ((pair0 + i % n_pairs) * 64 < S.rows)
+                    reinterpret_cast<float *>(A.rows_out + static_cast<int64_t>(A.jobs[joff + j0 + i / n_pairs]) * A.out_lay.stride() +
+                                              A.out_lay.da_offset())[pair0 + i % n_pairs] = nan;
+        }
+        return;
+    }
+
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int lr = lane & 15, q = lane >> 4;
+    const int nb = S.nb, groups = nb / 8, tail = nb % 8;
+    const int n_groups = groups + (tail ? 1 : 0), n_chunks = (nb + 3) / 4;
+    const int pair = pair0 + (wide ? wave : wave & 1);
+    const bool pair_live = pair * 64 < S.rows;
+    const bool two_tiles = pair * 64 + 32 < S.rows;          // the last pair may be one tile
+    const int split = 16 * ((live + 31) / 32);
+    const int wj = wide || wave < 2 ? 0 : split;
+    const int wend = wide || wave >= 2 ? live : (split < live ? split : live);
+    const int nf = pair_live && wend > wj ? (wend - wj + 15) / 16 : 0;   // live fragment columns, 0..4
+    const uint8_t * slot_base = A.bank + static_cast<size_t>(slot) * S.slot_bytes;
+
+    // weight stream: a buffer descriptor over the pair's codes (a dead pair reads the unit's first pair
+    // and drops it; a missing second tile reads the first)
+    const int src_pair = pair_live ? pair : pair0;
+    const int tile1 = __builtin_amdgcn_readfirstlane(src_pair * 64 + 32 < S.rows ? 1 : 0);   // index of fragments 2, 3's tile
+    const int code_tile = 32 * nb * 16, meta_tile = 32 * nb;
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr(const_cast<uint8_t *>(slot_base + static_cast<size_t>(src_pair) * 2 * code_tile)), static_cast<short>(0),
+        __builtin_amdgcn_readfirstlane((1 + tile1) * code_tile), 0x00020000);
+    const uint8_t * exp_base = slot_base + S.codes_bytes + static_cast<size_t>(src_pair) * 2 * meta_tile;
+    // A full group holds 16 bytes of codes per (slice, row) and 8 exponent bytes per row, the tail's 2, 4
+    // or 6 blocks 2 tail and tail bytes. The tail takes the same code loads with its own lane stride:
+    // what they read past a row's entry is not used (past the descriptor: zeros).
+    auto load_group = [&](int g, MxGroupRegs & w) {
+        const int cs = g < groups ? 16 : 2 * tail;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int so = (i >> 1) * tile1 * code_tile + g * 4096;
+            w.c[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rc, (2 * q * 32 + 16 * (i & 1) + lr) * cs, so, 0);
+            w.c[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rc, ((2 * q + 1) * 32 + 16 * (i & 1) + lr) * cs, so, 0);
+        }
+    };
+    // The loads of `w` are complete (an lds_dma_wait<0> came before): a use that takes the compiler's
+    // own wait for them here, where it costs nothing. At their first real use, behind the next
+    // stage's DMA, that wait would be for the DMA too.
+    auto landed = [&](MxGroupRegs & w) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(w.c[i][0]), "+v"(w.c[i][1]));
+    };
+    // Fold check over every exponent of the wave's rows (4 KiB at most).
+    unsigned unfold = 0;
+    for (int o = lane * 16; o < (1 + tile1) * meta_tile; o += 1024) {
+        const u32x4g m = *reinterpret_cast<const u32x4g *>(exp_base + o);
+        unfold |= mx_unfoldable(m[0]) | mx_unfoldable(m[1]) | mx_unfoldable(m[2]) | mx_unfoldable(m[3]);
+    }
+
+    // activation stages: DMA k = wave + 4i (1 KiB) holds jobs 4k..4k+3; the 16-byte part p = 4b + q of
+    // a job's 256 bytes sits at part p ^ (job & 15), so that a fragment read (16 jobs, one part)
+    // covers all banks. A load whose jobs are all past the tile's live ones is skipped; a dead job
+    // in a load with a live one reads the tile's first job.
+    auto row_off16 = [&](int jl) -> uint32_t {               // row offset of live local job jl, in 16-byte units
+        const int jb = A.jobs[joff + j0 + jl];
+        const int64_t row = A.b_ne1 == 1 ? jb / A.n_ids : jb;
+        return static_cast<uint32_t>(row * (A.lay.stride() / 16));
+    };
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+    const int part = (lane & 15) ^ ((4 * wave + (lane >> 4)) & 15);   // 4k = 4 wave (mod 16): one part for every load
+    uint32_t arow[8];                                        // row and part, in 16-byte units
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int jl = 4 * (wave + 4 * i) + (lane >> 4);
+        arow[i] = 4 * (wave + 4 * i) < live ? row_off16(jl < live ? jl : 0) + part : 0u;
+    }
+    const int djob = 64 * (wave & 1) + lane;
+    const uint32_t drow = row_off16(djob < live ? djob : 0);
+    const uint8_t * da_base = A.rows_in + A.lay.da_offset();
+    // Byte address of 16-byte unit `off` from `base`; opaque, so that the 64-bit offsets are not kept in
+    // registers over the K loop (spilled, their reloads waited for the DMA in flight).
+    auto unit_ptr = [](const uint8_t * base, uint32_t off) {
+        asm volatile("" : "+v"(off));
+        return base + static_cast<uint64_t>(off) * 16;
+    };
+    auto dma_stage = [&](int c) {
+        const uint32_t sb = lds0 + L::OFF_ACT + (c & 1) * L::ACT;
+        const uint8_t * base = A.rows_in + static_cast<int64_t>(c) * L::ROW;
+        const uint32_t back = 4 * c + 2 < nb ? 0 : part & 8; // the last stage of nb = 4n + 2 blocks holds two
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int k = wave + 4 * i;
+            if (4 * k < live) lds_dma_x4(unit_ptr(base, arow[i] - back), sb + k * 1024);
+        }
+        if (wave < 2 && 64 * wave < live) lds_dma_x4(unit_ptr(da_base, drow + c), lds0 + (c & 1) * L::DA + wave * 1024);
+    };
+
+    // the wave's exponents of group g: lanes 0..15 / 16..31 bring the 256 bytes of its two tiles (the
+    // tail's 32 tail bytes)
+    auto dma_exps = [&](int g) {
+        if (lane < 32 && (lane & 15) * 16 < 32 * (g < groups ? 8 : tail))
+            lds_dma_x4(exp_base + (lane >> 4) * tile1 * meta_tile + g * 256 + (lane & 15) * 16,
+                       lds0 + L::OFF_EXP + ((g & 1) * 4 + wave) * 512);
+    };
+
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jh = 0; jh < 4; ++jh) acc[i][jh] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bool flagged = false;                                    // wave-uniform: a live job holds -128 codes
+    if constexpr (FLAGGED) {
+        int f = 0;
+        if (lane < wend - wj)
+            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(wj + lane)) * 16 + A.lay.flag_offset());
+        flagged = __any(f != 0);
+    }
+
+    // K loop over NF live fragment columns; GENERAL: the general path (see above).
+    auto k_loop = [&](auto nf_c, auto general_c) {
+        constexpr int NF = decltype(nf_c)::value;
+        constexpr bool GENERAL = decltype(general_c)::value;
+        // this lane's part of block 0 of fragment column 0 (wj is a multiple of 16); block bb's is at
+        // the address with bits 6..7 flipped by bb (recomputed from an opaque copy at each use, a
+        // register less per block)
+        const uint32_t act0 = static_cast<uint32_t>((wj + lr) * L::ROW + ((q ^ lr) << 4));
+        // Blocks 4H .. of group g, its weights in w, its activations in stage H (nblk: 4, or 2 at the end
+        // of a row); TAIL: exponents packed by tail bytes per row.
+        auto half_group = [&](auto h_c, auto tail_c, int g, const MxGroupRegs & w, int nblk) {
+            constexpr int H = decltype(h_c)::value;
+            constexpr bool TAIL = decltype(tail_c)::value;
+            const uint8_t * exps = lds + L::OFF_EXP + ((g & 1) * 4 + wave) * 512;
+            auto exp_dword = [&](int i, int r) -> unsigned {   // row r of fragment i
+                if constexpr (!TAIL) return *reinterpret_cast<const unsigned *>(exps + i * 128 + r * 8 + 4 * H);
+                const uint16_t * p = reinterpret_cast<const uint16_t *>(exps + (i >> 1) * 256 + (16 * (i & 1) + r) * tail + 4 * H);
+                return static_cast<unsigned>(p[0]) | (static_cast<unsigned>(p[1]) << 16);
+            };
+            f32x4 da[NF];
+#pragma unroll
+            for (int jh = 0; jh < NF; ++jh)
+                da[jh] = *reinterpret_cast<const f32x4 *>(lds + H * L::DA + (wj + 16 * jh + lr) * 16);
+            uint32_t ablk = act0;
+            auto act = [&](int jh, int bb) {
+                return *reinterpret_cast<const half8_t *>(lds + L::OFF_ACT + H * L::ACT + jh * 16 * L::ROW + (ablk ^ (bb << 6)));
+            };
+            if constexpr (!GENERAL) {
+                unsigned ew[4];                              // raw e8m0 bytes of the half's four blocks
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ew[i] = exp_dword(i, lr) ^ 0x80808080u;
+                auto weights = [&](int i, int bb) {
+                    const float sc = __builtin_bit_cast(float, ((ew[i] >> (8 * bb)) & 0xFFu) << 23);   // 2^(e+1)
+                    return mx_a_operand(w.c[i][0][2 * H + (bb >> 1)], w.c[i][1][2 * H + (bb >> 1)], bb & 1, sc);
+                };
+                // Software pipeline over the (block, column) steps: fragment i's product of the previous
+                // step is summed right before its register takes this step's MFMA (a matrix result is
+                // some 16 cycles away; left to itself the compiler waits for each). A step also reads the
+                // next step's activation operand and, at a block's last column, converts the next
+                // block's weights.
+                half8_t a_op[4], bv[2];
+                f32x4 d[4];
+                bv[0] = act(0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) a_op[i] = weights(i, 0);
+                auto sum = [&](int t, int i) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][t % NF][j] = __builtin_fmaf(da[t % NF][t / NF], d[i][j], acc[i][t % NF][j]);
+                };
+#pragma unroll
+                for (int t = 0; t < 4 * NF; ++t) {
+                    if (t == 2 * NF && nblk <= 2) break;
+                    if ((t + 1) % NF == 0) asm volatile("" : "+v"(ablk));
+                    if (t + 1 < 4 * NF) bv[(t + 1) & 1] = act((t + 1) % NF, (t + 1) / NF);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (t > 0) sum(t - 1, i);
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op[i], bv[t & 1], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        if (t % NF == NF - 1 && t / NF < 3) a_op[i] = weights(i, t / NF + 1);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // the activation read
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (t > 0) __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);             // the sums,
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                        // one MFMA,
+                        if (t % NF == NF - 1) __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);  // the conversion
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (nblk <= 2) sum(2 * NF - 1, i);
+                    else sum(4 * NF - 1, i);
+                }
+                // keeps the sums in this place: moved past the branches that follow the half group, they
+                // would hold every block's products in registers
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int jh = 0; jh < NF; ++jh) asm volatile("" : "+v"(acc[i][jh]));
+            } else {
+#pragma clang loop unroll(disable)
+                for (int bb = 0; bb < nblk; ++bb) {
+                    half8_t bv[NF];
+                    float dv[NF];
+#pragma unroll
+                    for (int jh = 0; jh < NF; ++jh) {
+                        bv[jh] = act(jh, bb);
+                        dv[jh] = bb == 0 ? da[jh][0] : (bb == 1 ? da[jh][1] : (bb == 2 ? da[jh][2] : da[jh][3]));
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const unsigned w0 = bb < 2 ? w.c[i][0][2 * H] : w.c[i][0][2 * H + 1];
+                        const unsigned w1 = bb < 2 ? w.c[i][1][2 * H] : w.c[i][1][2 * H + 1];
+                        const half8_t a_op = mx_a_operand(w0 >> (16 * (bb & 1)), w1 >> (16 * (bb & 1)), 0);
+                        int e[4];                            // exponents of output rows 16i + 4q + j
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            e[j] = static_cast<signed char>(exp_dword(i, 4 * q + j) >> (8 * bb));
+#pragma unroll
+                        for (int jh = 0; jh < NF; ++jh) {
+                            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op, bv[jh], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                            if constexpr (FLAGGED)
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(neg_part(a_op), is_neg128_x256(bv[jh]), d, 0, 0, 0);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                acc[i][jh][j] = __builtin_fmaf(__builtin_amdgcn_ldexpf(dv[jh], e[j]), d[j], acc[i][jh][j]);
+                        }
+                    }
+                }
+            }
+        };
+        constexpr std::integral_constant<int, 0> h0{};
+        constexpr std::integral_constant<int, 1> h1{};
+        // One full group: its weights are in `cur`; the next group's loads go into `nxt` (past the last
+        // group: the last one's again, so that the loads have no branch around them and the
+        // compiler's wait counts stay exact). The DMA of the next stage is issued first and the
+        // weight loads after it, so the wait for the DMA leaves them in flight across the first
+        // barrier.
+        auto group_step = [&](int g, const MxGroupRegs & cur, MxGroupRegs & nxt) {
+            dma_stage(2 * g + 1);
+            const bool next = g + 1 < n_groups;
+            if (next) dma_exps(g + 1);
+            load_group(__builtin_amdgcn_readfirstlane(next ? g + 1 : g), nxt);
+            half_group(h0, std::false_type{}, g, cur, 4);
+            lds_dma_wait<kMxGroupLoads>();
+            __syncthreads();
+            if (next) dma_stage(2 * g + 2);
+            half_group(h1, std::false_type{}, g, cur, 4);
+            lds_dma_wait<0>();
+            landed(nxt);
+            __syncthreads();
+        };
+        MxGroupRegs wa, wb;
+        dma_exps(0);
+        load_group(0, wa);
+        lds_dma_wait<0>();
+        landed(wa);
+        __syncthreads();
+#pragma clang loop unroll(disable)
+        for (int g = 0; g < groups; g += 2) {
+            group_step(g, wa, wb);
+            if (g + 1 < groups) {
+                group_step(g + 1, wb, wa);
+            } else {
+                wa = wb;
+            }
+        }
+        if (tail) {   // 2, 4 or 6 blocks: one stage, or one and a half
+            if (tail == 6) dma_stage(2 * groups + 1);
+            half_group(h0, std::true_type{}, groups, wa, tail < 4 ? tail : 4);
+            if (tail == 6) {
+                lds_dma_wait<0>();
+                __syncthreads();
+                half_group(h1, std::true_type{}, groups, wa, 2);
+            }
+        }
+    };
+    dma_stage(0);
+    // Waves may take different instantiations: each issues the same stage loads and reaches the same
+    // number of barriers.
+    const bool general = __any(unfold != 0) || flagged;
+    if (nf == 0) {
+        lds_dma_wait<0>();
+        __syncthreads();
+        for (int c = 1; c < n_chunks; ++c) {
+            dma_stage(c);
+            lds_dma_wait<0>();
+            __syncthreads();
+        }
+        if (n_chunks == 2 * groups) __syncthreads();
+        return;
+    }
+    constexpr std::false_type fold{};
+    if (general) k_loop(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (nf == 4) k_loop(std::integral_constant<int, 4>{}, fold);
+    else if (nf == 3) k_loop(std::integral_constant<int, 3>{}, fold);
+    else if (nf == 2) k_loop(std::integral_constant<int, 2>{}, fold);
+    else k_loop(std::integral_constant<int, 1>{}, fold);
+
+    // Epilogue, from registers: lane (q, lr) holds rows 16i + 4q .. + 3 of the pair for job
+    // wj + 16jh + lr. Biases (ggml row order), then fp32 rows (times the routing weight when given)
+    // as one 16-byte store per fragment, or GLU + Q8_0 requantization: fragments 0 / 1 and 2 / 3 are
+    // the gate / up rows of the block's elements 4q .. + 3 and 16 + 4q .. + 3.
+    float bias[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool row_live = i < 2 || two_tiles;
+        const int64_t grow = ggml_row(static_cast<int64_t>(pair) * 64 + 16 * i + 4 * q, S.rows, S.interleave);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias[i][j] = A.bias && row_live ? A.bias[static_cast<size_t>(expert) * S.rows + grow + j] : 0.0f;
+    }
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) {
+        const int jl = wj + 16 * jh + lr;
+        if (jh >= nf) break;
+        const bool jlive = jl < wend;
+        const int job = jlive ? A.jobs[joff + j0 + jl] : 0;
+        if constexpr (EPI == 0) {
+            const float rs = A.row_scale && jlive ? A.row_scale[job] : 1.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!jlive || (i >= 2 && !two_tiles)) continue;
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[j] = acc[i][jh][j];
+                    if (A.bias) v[j] = v[j] + bias[i][j];
+                    if (A.row_scale) v[j] = v[j] * rs;
+                }
+                // aligned runs of 4 device rows are 4 consecutive ggml rows, also in interleaved banks
+                float * out = A.dst + static_cast<size_t>(job) * S.rows +
+                              ggml_row(static_cast<int64_t>(pair) * 64 + 16 * i + 4 * q, S.rows, S.interleave);
+                if (A.dst_vec4) {
+                    *reinterpret_cast<float4 *>(out) = float4{v[0], v[1], v[2], v[3]};
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) out[j] = v[j];
+                }
+            }
+        } else {
+            float x[2][4], amax = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float gv = acc[2 * t][jh][j], uv = acc[2 * t + 1][jh][j];
+                    if (A.bias) gv = gv + bias[2 * t][j], uv = uv + bias[2 * t + 1][j];
+                    x[t][j] = glu_fast(A.activation, gv, uv, A.alpha, A.limit);
+                    amax = fmaxf(amax, fabsf(x[t][j]));
+                }
+            amax = fmaxf(amax, __shfl_xor(amax, 16));        // the block's other lanes of this job
+            amax = fmaxf(amax, __shfl_xor(amax, 32));
+            const float d = amax / 127.0f;
+            const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+            if (!jlive) continue;
+            uint8_t * out = A.rows_out + static_cast<int64_t>(job) * A.out_lay.stride();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                half4_g c;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v = rintf(x[t][j] * id);
+                    v = v > 127.0f ? 127.0f : (v < -128.0f ? -128.0f : v);
+                    c[j] = static_cast<_Float16>(v);
+                }
+                *reinterpret_cast<half4_g *>(out + (static_cast<int64_t>(pair) * 32 + 16 * t + 4 * q) * 2) = c;
+            }
+            if (q == 0) {
+                reinterpret_cast<float *>(out + A.out_lay.da_offset())[pair] = static_cast<float>(static_cast<_Float16>(d));
+                if (pair == 0) *reinterpret_cast<int *>(out + A.out_lay.flag_offset()) = 0;   // never -128
+            }
+        }
+    }
+}
+
 // Tiles of job_tile jobs per active expert, in active order: one workgroup, wave scans plus a
 // scan of the 16 wave totals.
 __global__ __launch_bounds__(1024) void gemm_tiles_kernel(const int32_t * counts, const int32_t * active,
@@ -993,6 +1449,16 @@ __global__ __launch_bounds__(256) void gemm_rows_from_q8_kernel(const uint8_t * 
     if (neg) atomicOr(&s_flag, 1);
     __syncthreads();
     if (threadIdx.x == 0) *reinterpret_cast<int *>(o + L.flag_offset()) = s_flag;
+}
+
+template <int EPI, bool FLAGGED>
+void launch_mx_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
+    GemmArgs b = a;
+    b.row_units = static_cast<int>((rows + 127) / 128);
+    const int64_t items = static_cast<int64_t>(b.row_units) * max_tiles;
+    hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)), dim3(kGemmThreads), 0,
+                       stream, b);
+    check_hip(hipGetLastError(), "grouped GEMM launch");
 }
 
 template <int TYPE, int EPI, bool FLAGGED>
@@ -1373,9 +1839,9 @@ void launch_grouped_gemm(const GemmParams & p, hipStream_t stream) {
     require(p.grid_tiles >= 0 && (p.grid_tiles == 0 || p.tile_filter != nullptr), "grid tile bound needs a tile filter");
     const int mt = static_cast<int>(p.grid_tiles > 0 ? std::min<int64_t>(p.grid_tiles, max_tiles) : max_tiles);
     if (bank.type == VBM_TYPE_MXFP4) {
-        if (p.flagged_rows) launch_gemm_typed<39, 0, true>(a, row_pairs, mt, stream);
-        else if (p.epilogue == 0) launch_gemm_typed<39, 0, false>(a, row_pairs, mt, stream);
-        else launch_gemm_typed<39, 1, false>(a, row_pairs, mt, stream);
+        if (p.flagged_rows) launch_mx_rows_gemm<0, true>(a, bank.rows, mt, stream);
+        else if (p.epilogue == 0) launch_mx_rows_gemm<0, false>(a, bank.rows, mt, stream);
+        else launch_mx_rows_gemm<1, false>(a, bank.rows, mt, stream);
     } else {
         if (p.flagged_rows) launch_gemm_typed<8, 0, true>(a, row_pairs, mt, stream);
         else if (p.epilogue == 0) launch_gemm_typed<8, 0, false>(a, row_pairs, mt, stream);
