@@ -89,7 +89,7 @@ struct GemmArgs {
     const float * row_scale;   // epilogue 0: per-job factor applied after the bias (routing weights), or null
     float * dst;               // epilogue 0: [job][rows]
     int row_pairs;             // 64-row tile pairs of the bank
-    int row_units;             // MXFP4: 128-row units of the bank
+    int row_units;             // MXFP4: 256-row units of the bank
     uint8_t * rows_out;        // epilogue 1: GLU output rows for the down projection (out_lay)
     GemmRowLayout out_lay;
     int activation;
@@ -870,12 +870,9 @@ __global__ __launch_bounds__(kGemmThreads, (TYPE == 8 && !FLAGGED) ? 3 : 1) void
 // up to 64 jobs: a 4 x 4 grid of 16 x 16 fragments. Its weights go from the bank straight into
 // registers, one 8-block group ahead (no other wave of the workgroup needs them; as A operand, lane
 // (q, r) of a fragment takes the 16-byte entries of slices 2q and 2q + 1 of its row as stored), and
-// only the activation rows, which every wave reads, are staged in LDS. A workgroup (4 waves) takes
-//   - job tiles of at most 64 live jobs: four tile pairs (256 rows) x the tile, so the activation
-//     rows are fetched once per 256 rows;
-//   - larger ones (up to 128): two tile pairs x two halves of the live jobs, split at a multiple of 16.
-// Stages hold four blocks (half a bank group) of every live job's codes and block scales, two of
-// them in turn, so one wait and one barrier per four blocks.
+// only the activation rows, which the workgroup's four waves all read, are staged in LDS: a stage is a
+// bank group (eight blocks) of the codes and block scales of up to 64 jobs, two of them in turn, so
+// one wait and one barrier per group. A workgroup takes 256 rows x one job tile.
 // Each wave's block products are summed with one FMA per output and block in block order, as in
 // every form of this kernel: the split over waves changes no bit of the result.
 //
@@ -884,20 +881,19 @@ __global__ __launch_bounds__(kGemmThreads, (TYPE == 8 && !FLAGGED) ? 3 : 1) void
 // first; otherwise, and for waves holding -128 codes (FLAGGED), the wave takes the general path:
 // doubled-integer operands, ldexp(d_act, e) per output, and the exact -128 correction.
 struct MxStageLayout {
-    static constexpr int kJobs = 128, CB = 4;
-    static constexpr int ROW = CB * 64;                        // f16 codes of a job and stage
-    static constexpr int DA = kJobs * CB * 4;                  // [job][4 blocks] fp32 block scales, both stages first
-    static constexpr int OFF_EXP = 2 * DA;                     // [group & 1][wave][64 rows] x 8 exponent bytes
-    static constexpr int OFF_ACT = OFF_EXP + 2 * 4 * 512;      // (last: every LDS read then has a 16-bit offset)
-    static constexpr int ACT = kJobs * ROW;
-    static constexpr int BYTES = OFF_ACT + 2 * ACT;
+    static constexpr int kJobs = 64;
+    static constexpr int ROW = 8 * 64;                         // f16 codes of a job and stage
+    static constexpr int DA = kJobs * 8 * 4;                   // [job][8 blocks] fp32 block scales, both stages first
+    static constexpr int OFF_ACT = 2 * DA, ACT = kJobs * ROW;  // (every fragment read then has a 16-bit offset)
+    static constexpr int OFF_EXP = OFF_ACT + 2 * ACT;          // [stage][wave][64 rows] x 8 exponent bytes
+    static constexpr int OFF_ROW = OFF_EXP + 2 * 4 * 512;      // [job] row offset in 16-byte units
+    static constexpr int BYTES = OFF_ROW + kJobs * 4;
 };
 // Weights of a wave and group: entry [i][s] is slice 2q + s of row 16i + lr (dword d holds blocks
 // 2d, 2d + 1). Their exponents are staged in LDS: as registers too they would spill.
 struct MxGroupRegs {
     u32x4g c[4][2];
 };
-constexpr int kMxGroupLoads = 8;   // vector loads of a group
 
 // Every stored exponent byte (signed e) of the dword in [-14, 12]: e + 14 and e + 19 both in [0, 32).
 __device__ __forceinline__ unsigned mx_unfoldable(unsigned w) {
@@ -917,7 +913,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
     if (slot8 >= per_xcd || item >= n_items) return;
     const int ti = item / A.row_units;
-    const int unit = item - ti * A.row_units;          // 128 rows; 256 for tiles of at most 64 jobs
+    const int unit = item - ti * A.row_units;
     const int expert = cst<int32_t>(A.tile_expert)[ti];
     const int j0 = cst<int32_t>(A.tile_start)[ti];
     const int count = cst<int32_t>(A.counts)[expert];
@@ -925,9 +921,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     const int slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[expert] : expert;
     const GemmShape S = A.shape;
     const int live = count - j0 < L::kJobs ? count - j0 : L::kJobs;
-    const bool wide = live <= 64;
-    const int pair0 = unit * (wide ? 4 : 2), n_pairs = wide ? 4 : 2;
-    if (pair0 * 64 >= S.rows) return;
+    const int pair0 = unit * 4, n_pairs = 4;
     if (slot < 0 || slot >= S.n_slots) {
         // Expert not resident in this bank: NaN outputs, as in the decode kernels (a tile filter
         // removes the experts a pass skips on purpose, so this is a bad map).
@@ -950,14 +944,11 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int lr = lane & 15, q = lane >> 4;
     const int nb = S.nb, groups = nb / 8, tail = nb % 8;
-    const int n_groups = groups + (tail ? 1 : 0), n_chunks = (nb + 3) / 4;
-    const int pair = pair0 + (wide ? wave : wave & 1);
+    const int n_groups = groups + (tail ? 1 : 0);
+    const int pair = pair0 + wave;
     const bool pair_live = pair * 64 < S.rows;
     const bool two_tiles = pair * 64 + 32 < S.rows;          // the last pair may be one tile
-    const int split = 16 * ((live + 31) / 32);
-    const int wj = wide || wave < 2 ? 0 : split;
-    const int wend = wide || wave >= 2 ? live : (split < live ? split : live);
-    const int nf = pair_live && wend > wj ? (wend - wj + 15) / 16 : 0;   // live fragment columns, 0..4
+    const int nf = pair_live ? (live + 15) / 16 : 0;         // live fragment columns, 0..4
     const uint8_t * slot_base = A.bank + static_cast<size_t>(slot) * S.slot_bytes;
 
     // weight stream: a buffer descriptor over the pair's codes (a dead pair reads the unit's first pair
@@ -972,7 +963,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     // A full group holds 16 bytes of codes per (slice, row) and 8 exponent bytes per row, the tail's 2, 4
     // or 6 blocks 2 tail and tail bytes. The tail takes the same code loads with its own lane stride:
     // what they read past a row's entry is not used (past the descriptor: zeros).
-    auto load_group = [&](int g, MxGroupRegs & w) {
+    auto load_group = [&](int g, MxGroupRegs & w) __attribute__((always_inline)) {
         const int cs = g < groups ? 16 : 2 * tail;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -984,58 +975,63 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     // The loads of `w` are complete (an lds_dma_wait<0> came before): a use that takes the compiler's
     // own wait for them here, where it costs nothing. At their first real use, behind the next
     // stage's DMA, that wait would be for the DMA too.
-    auto landed = [&](MxGroupRegs & w) {
+    auto landed = [&](MxGroupRegs & w) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(w.c[i][0]), "+v"(w.c[i][1]));
     };
-    // Fold check over every exponent of the wave's rows (4 KiB at most).
+    // Fold check over every exponent of the wave's rows (k <= 4096: 8 KiB at most; all loads in flight
+    // together).
     unsigned unfold = 0;
-    for (int o = lane * 16; o < (1 + tile1) * meta_tile; o += 1024) {
-        const u32x4g m = *reinterpret_cast<const u32x4g *>(exp_base + o);
-        unfold |= mx_unfoldable(m[0]) | mx_unfoldable(m[1]) | mx_unfoldable(m[2]) | mx_unfoldable(m[3]);
+    {
+        u32x4g m[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int o = lane * 16 + i * 1024;
+            m[i] = *reinterpret_cast<const u32x4g *>(exp_base + (o < (1 + tile1) * meta_tile ? o : 0));
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) unfold |= mx_unfoldable(m[i][0]) | mx_unfoldable(m[i][1]) | mx_unfoldable(m[i][2]) | mx_unfoldable(m[i][3]);
     }
 
-    // activation stages: DMA k = wave + 4i (1 KiB) holds jobs 4k..4k+3; the 16-byte part p = 4b + q of
-    // a job's 256 bytes sits at part p ^ (job & 15), so that a fragment read (16 jobs, one part)
-    // covers all banks. A load whose jobs are all past the tile's live ones is skipped; a dead job
-    // in a load with a live one reads the tile's first job.
-    auto row_off16 = [&](int jl) -> uint32_t {               // row offset of live local job jl, in 16-byte units
-        const int jb = A.jobs[joff + j0 + jl];
-        const int64_t row = A.b_ne1 == 1 ? jb / A.n_ids : jb;
-        return static_cast<uint32_t>(row * (A.lay.stride() / 16));
+    // activation stages: DMA k = wave + 4i (1 KiB) holds jobs 2k, 2k + 1; the 16-byte part p = 4b + q of a
+    // job's 512 bytes sits at part p ^ (job & 15), so that a fragment read (16 jobs, one part) covers
+    // all banks. A load whose jobs are all past the tile's live ones is skipped; a dead job in a load
+    // with a live one reads the tile's first job.
+    auto row_off16 = [&](int jl) __attribute__((always_inline)) -> uint32_t {               // row offset of live local job jl, in 16-byte units
+        const uint32_t jb = static_cast<uint32_t>(A.jobs[joff + j0 + jl]);
+        const uint32_t row = A.b_ne1 == 1 ? jb / static_cast<uint32_t>(A.n_ids) : jb;
+        return row * static_cast<uint32_t>(A.lay.stride() / 16);
     };
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-    const int part = (lane & 15) ^ ((4 * wave + (lane >> 4)) & 15);   // 4k = 4 wave (mod 16): one part for every load
-    uint32_t arow[8];                                        // row and part, in 16-byte units
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int jl = 4 * (wave + 4 * i) + (lane >> 4);
-        arow[i] = 4 * (wave + 4 * i) < live ? row_off16(jl < live ? jl : 0) + part : 0u;
-    }
-    const int djob = 64 * (wave & 1) + lane;
-    const uint32_t drow = row_off16(djob < live ? djob : 0);
+    const int part = (lane & 31) ^ (2 * wave + (lane >> 5)); // of the loads with even i; odd i flip bit 3 (2k mod 16)
+    const int djob = 32 * (wave & 1) + (lane >> 1);          // block scales: waves 0 and 1, 32 jobs x 32 bytes
     const uint8_t * da_base = A.rows_in + A.lay.da_offset();
-    // Byte address of 16-byte unit `off` from `base`; opaque, so that the 64-bit offsets are not kept in
-    // registers over the K loop (spilled, their reloads waited for the DMA in flight).
-    auto unit_ptr = [](const uint8_t * base, uint32_t off) {
-        asm volatile("" : "+v"(off));
-        return base + static_cast<uint64_t>(off) * 16;
-    };
-    auto dma_stage = [&](int c) {
-        const uint32_t sb = lds0 + L::OFF_ACT + (c & 1) * L::ACT;
-        const uint8_t * base = A.rows_in + static_cast<int64_t>(c) * L::ROW;
-        const uint32_t back = 4 * c + 2 < nb ? 0 : part & 8; // the last stage of nb = 4n + 2 blocks holds two
+    uint32_t * row_tab = reinterpret_cast<uint32_t *>(lds + L::OFF_ROW);
+    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
+    __syncthreads();
+    // (the rows' offsets are read back from LDS by every group: kept in registers they would spill, and
+    // the spills' reloads wait for the DMA in flight)
+    auto dma_stage = [&](int g) __attribute__((always_inline)) {
+        const uint32_t sb = lds0 + L::OFF_ACT + (g & 1) * L::ACT;
+        const uint8_t * base = A.rows_in + static_cast<int64_t>(g) * L::ROW;
+        uint32_t row[8], drow = row_tab[djob];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) row[i] = row_tab[2 * (wave + 4 * i) + (lane >> 5)];
+        // the tail's stage: parts past its blocks read one of the first two blocks' again
+        const int parts = g < groups ? 32 : 4 * tail;
+        const uint32_t pe = part < parts ? part : part & 7, po = (part ^ 8) < parts ? part ^ 8 : part & 7;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int k = wave + 4 * i;
-            if (4 * k < live) lds_dma_x4(unit_ptr(base, arow[i] - back), sb + k * 1024);
+            if (2 * k < live) lds_dma_x4(base + static_cast<uint64_t>(row[i] + (i & 1 ? po : pe)) * 16, sb + k * 1024);
         }
-        if (wave < 2 && 64 * wave < live) lds_dma_x4(unit_ptr(da_base, drow + c), lds0 + (c & 1) * L::DA + wave * 1024);
+        if (wave < 2 && 32 * wave < live)                    // (a tail of at most four blocks has no second 16 bytes)
+            lds_dma_x4(da_base + static_cast<uint64_t>(drow + 2 * g + (parts > 16 ? lane & 1 : 0)) * 16,
+                       lds0 + (g & 1) * L::DA + wave * 1024);
     };
-
     // the wave's exponents of group g: lanes 0..15 / 16..31 bring the 256 bytes of its two tiles (the
     // tail's 32 tail bytes)
-    auto dma_exps = [&](int g) {
+    auto dma_exps = [&](int g) __attribute__((always_inline)) {
         if (lane < 32 && (lane & 15) * 16 < 32 * (g < groups ? 8 : tail))
             lds_dma_x4(exp_base + (lane >> 4) * tile1 * meta_tile + g * 256 + (lane & 15) * 16,
                        lds0 + L::OFF_EXP + ((g & 1) * 4 + wave) * 512);
@@ -1049,26 +1045,26 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     bool flagged = false;                                    // wave-uniform: a live job holds -128 codes
     if constexpr (FLAGGED) {
         int f = 0;
-        if (lane < wend - wj)
-            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(wj + lane)) * 16 + A.lay.flag_offset());
+        if (lane < live)
+            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(lane)) * 16 + A.lay.flag_offset());
         flagged = __any(f != 0);
     }
 
     // K loop over NF live fragment columns; GENERAL: the general path (see above).
-    auto k_loop = [&](auto nf_c, auto general_c) {
+    auto k_loop = [&](auto nf_c, auto general_c) __attribute__((always_inline)) {
         constexpr int NF = decltype(nf_c)::value;
         constexpr bool GENERAL = decltype(general_c)::value;
-        // this lane's part of block 0 of fragment column 0 (wj is a multiple of 16); block bb's is at
-        // the address with bits 6..7 flipped by bb (recomputed from an opaque copy at each use, a
-        // register less per block)
-        const uint32_t act0 = static_cast<uint32_t>((wj + lr) * L::ROW + ((q ^ lr) << 4));
-        // Blocks 4H .. of group g, its weights in w, its activations in stage H (nblk: 4, or 2 at the end
-        // of a row); TAIL: exponents packed by tail bytes per row.
-        auto half_group = [&](auto h_c, auto tail_c, int g, const MxGroupRegs & w, int nblk) {
+        // this lane's part of block 0 of fragment column 0; block b's is at the address with bits 6..8
+        // flipped by b (recomputed from an opaque copy at each use, a register less per block)
+        const uint32_t act0 = static_cast<uint32_t>(lr * L::ROW + ((q ^ lr) << 4));
+        // Blocks 4H .. of group g (stage ST), its weights in w (nblk: 4, or 2 at the end of a row); TAIL:
+        // exponents packed by tail bytes per row. `issue` starts the next group's DMA and loads: the
+        // half's first LDS reads go out before it, so that they land while it issues.
+        auto half_group = [&](int ST, auto h_c, auto tail_c, const MxGroupRegs & w, int nblk, auto && issue) __attribute__((always_inline)) {
             constexpr int H = decltype(h_c)::value;
             constexpr bool TAIL = decltype(tail_c)::value;
-            const uint8_t * exps = lds + L::OFF_EXP + ((g & 1) * 4 + wave) * 512;
-            auto exp_dword = [&](int i, int r) -> unsigned {   // row r of fragment i
+            const uint8_t * exps = lds + L::OFF_EXP + (ST * 4 + wave) * 512;
+            auto exp_dword = [&](int i, int r) __attribute__((always_inline)) -> unsigned {   // row r of fragment i
                 if constexpr (!TAIL) return *reinterpret_cast<const unsigned *>(exps + i * 128 + r * 8 + 4 * H);
                 const uint16_t * p = reinterpret_cast<const uint16_t *>(exps + (i >> 1) * 256 + (16 * (i & 1) + r) * tail + 4 * H);
                 return static_cast<unsigned>(p[0]) | (static_cast<unsigned>(p[1]) << 16);
@@ -1076,16 +1072,23 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
             f32x4 da[NF];
 #pragma unroll
             for (int jh = 0; jh < NF; ++jh)
-                da[jh] = *reinterpret_cast<const f32x4 *>(lds + H * L::DA + (wj + 16 * jh + lr) * 16);
+                da[jh] = *reinterpret_cast<const f32x4 *>(lds + ST * L::DA + (16 * jh + lr) * 32 + 16 * H);
             uint32_t ablk = act0;
-            auto act = [&](int jh, int bb) {
-                return *reinterpret_cast<const half8_t *>(lds + L::OFF_ACT + H * L::ACT + jh * 16 * L::ROW + (ablk ^ (bb << 6)));
+            auto act = [&](int jh, int bb) __attribute__((always_inline)) {
+                return *reinterpret_cast<const half8_t *>(lds + L::OFF_ACT + ST * L::ACT + jh * 16 * L::ROW + (ablk ^ ((4 * H + bb) << 6)));
             };
             if constexpr (!GENERAL) {
+                constexpr int PB = 2;                        // activation operands read this many steps ahead
+                half8_t a_op[4], bv[PB + 1];
                 unsigned ew[4];                              // raw e8m0 bytes of the half's four blocks
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ew[i] = exp_dword(i, lr) ^ 0x80808080u;
-                auto weights = [&](int i, int bb) {
+                for (int i = 0; i < 4; ++i) ew[i] = exp_dword(i, lr);
+#pragma unroll
+                for (int t = 0; t < PB; ++t) bv[t] = act(t % NF, t / NF);
+                issue();
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ew[i] ^= 0x80808080u;
+                auto weights = [&](int i, int bb) __attribute__((always_inline)) {
                     const float sc = __builtin_bit_cast(float, ((ew[i] >> (8 * bb)) & 0xFFu) << 23);   // 2^(e+1)
                     return mx_a_operand(w.c[i][0][2 * H + (bb >> 1)], w.c[i][1][2 * H + (bb >> 1)], bb & 1, sc);
                 };
@@ -1094,12 +1097,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
                 // some 16 cycles away; left to itself the compiler waits for each). A step also reads the
                 // next step's activation operand and, at a block's last column, converts the next
                 // block's weights.
-                half8_t a_op[4], bv[2];
                 f32x4 d[4];
-                bv[0] = act(0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) a_op[i] = weights(i, 0);
-                auto sum = [&](int t, int i) {
+                auto sum = [&](int t, int i) __attribute__((always_inline)) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         acc[i][t % NF][j] = __builtin_fmaf(da[t % NF][t / NF], d[i][j], acc[i][t % NF][j]);
@@ -1107,12 +1108,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 #pragma unroll
                 for (int t = 0; t < 4 * NF; ++t) {
                     if (t == 2 * NF && nblk <= 2) break;
-                    if ((t + 1) % NF == 0) asm volatile("" : "+v"(ablk));
-                    if (t + 1 < 4 * NF) bv[(t + 1) & 1] = act((t + 1) % NF, (t + 1) / NF);
+                    if ((t + PB) % NF == 0) asm volatile("" : "+v"(ablk));
+                    if (t + PB < 4 * NF) bv[(t + PB) % (PB + 1)] = act((t + PB) % NF, (t + PB) / NF);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         if (t > 0) sum(t - 1, i);
-                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op[i], bv[t & 1], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op[i], bv[t % (PB + 1)], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
                         if (t % NF == NF - 1 && t / NF < 3) a_op[i] = weights(i, t / NF + 1);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // the activation read
@@ -1136,6 +1137,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 #pragma unroll
                     for (int jh = 0; jh < NF; ++jh) asm volatile("" : "+v"(acc[i][jh]));
             } else {
+                issue();
 #pragma clang loop unroll(disable)
                 for (int bb = 0; bb < nblk; ++bb) {
                     half8_t bv[NF];
@@ -1171,61 +1173,51 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
         constexpr std::integral_constant<int, 1> h1{};
         // One full group: its weights are in `cur`; the next group's loads go into `nxt` (past the last
         // group: the last one's again, so that the loads have no branch around them and the
-        // compiler's wait counts stay exact). The DMA of the next stage is issued first and the
-        // weight loads after it, so the wait for the DMA leaves them in flight across the first
-        // barrier.
-        auto group_step = [&](int g, const MxGroupRegs & cur, MxGroupRegs & nxt) {
-            dma_stage(2 * g + 1);
+        // compiler's wait counts stay exact).
+        auto group_step = [&](int st, int g, const MxGroupRegs & cur, MxGroupRegs & nxt) __attribute__((always_inline)) {
             const bool next = g + 1 < n_groups;
-            if (next) dma_exps(g + 1);
-            load_group(__builtin_amdgcn_readfirstlane(next ? g + 1 : g), nxt);
-            half_group(h0, std::false_type{}, g, cur, 4);
-            lds_dma_wait<kMxGroupLoads>();
-            __syncthreads();
-            if (next) dma_stage(2 * g + 2);
-            half_group(h1, std::false_type{}, g, cur, 4);
+            half_group(st, h0, std::false_type{}, cur, 4, [&] {
+                if (next) {
+                    dma_stage(g + 1);
+                    dma_exps(g + 1);
+                }
+                load_group(__builtin_amdgcn_readfirstlane(next ? g + 1 : g), nxt);
+            });
+            half_group(st, h1, std::false_type{}, cur, 4, [] {});
             lds_dma_wait<0>();
             landed(nxt);
             __syncthreads();
         };
         MxGroupRegs wa, wb;
-        dma_exps(0);
         load_group(0, wa);
         lds_dma_wait<0>();
         landed(wa);
         __syncthreads();
 #pragma clang loop unroll(disable)
         for (int g = 0; g < groups; g += 2) {
-            group_step(g, wa, wb);
-            if (g + 1 < groups) {
-                group_step(g + 1, wb, wa);
-            } else {
-                wa = wb;
-            }
+            group_step(0, g, wa, wb);
+            if (g + 1 < groups) group_step(1, g + 1, wb, wa);
+            else wa = wb;
         }
-        if (tail) {   // 2, 4 or 6 blocks: one stage, or one and a half
-            if (tail == 6) dma_stage(2 * groups + 1);
-            half_group(h0, std::true_type{}, groups, wa, tail < 4 ? tail : 4);
-            if (tail == 6) {
-                lds_dma_wait<0>();
-                __syncthreads();
-                half_group(h1, std::true_type{}, groups, wa, 2);
-            }
+        if (tail) {   // 2, 4 or 6 blocks
+            half_group(groups & 1, h0, std::true_type{}, wa, tail < 4 ? tail : 4, [] {});
+            if (tail == 6) half_group(groups & 1, h1, std::true_type{}, wa, 2, [] {});
         }
     };
     dma_stage(0);
+    dma_exps(0);
     // Waves may take different instantiations: each issues the same stage loads and reaches the same
     // number of barriers.
     const bool general = __any(unfold != 0) || flagged;
     if (nf == 0) {
         lds_dma_wait<0>();
         __syncthreads();
-        for (int c = 1; c < n_chunks; ++c) {
-            dma_stage(c);
+        for (int g = 1; g < n_groups; ++g) {
+            dma_stage(g);
             lds_dma_wait<0>();
             __syncthreads();
         }
-        if (n_chunks == 2 * groups) __syncthreads();
+        if (!tail) __syncthreads();
         return;
     }
     constexpr std::false_type fold{};
@@ -1236,7 +1228,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     else k_loop(std::integral_constant<int, 1>{}, fold);
 
     // Epilogue, from registers: lane (q, lr) holds rows 16i + 4q .. + 3 of the pair for job
-    // wj + 16jh + lr. Biases (ggml row order), then fp32 rows (times the routing weight when given)
+    // 16jh + lr. Biases (ggml row order), then fp32 rows (times the routing weight when given)
     // as one 16-byte store per fragment, or GLU + Q8_0 requantization: fragments 0 / 1 and 2 / 3 are
     // the gate / up rows of the block's elements 4q .. + 3 and 16 + 4q .. + 3.
     float bias[4][4];
@@ -1247,14 +1239,19 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 #pragma unroll
         for (int j = 0; j < 4; ++j) bias[i][j] = A.bias && row_live ? A.bias[static_cast<size_t>(expert) * S.rows + grow + j] : 0.0f;
     }
+    int jobs[4];
+    float scales[4];
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) jobs[jh] = A.jobs[joff + j0 + (16 * jh + lr < live ? 16 * jh + lr : 0)];
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) scales[jh] = EPI == 0 && A.row_scale ? A.row_scale[jobs[jh]] : 1.0f;
 #pragma unroll
     for (int jh = 0; jh < 4; ++jh) {
-        const int jl = wj + 16 * jh + lr;
         if (jh >= nf) break;
-        const bool jlive = jl < wend;
-        const int job = jlive ? A.jobs[joff + j0 + jl] : 0;
+        const bool jlive = 16 * jh + lr < live;
+        const int job = jobs[jh];
         if constexpr (EPI == 0) {
-            const float rs = A.row_scale && jlive ? A.row_scale[job] : 1.0f;
+            const float rs = scales[jh];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (!jlive || (i >= 2 && !two_tiles)) continue;
@@ -1454,7 +1451,7 @@ __global__ __launch_bounds__(256) void gemm_rows_from_q8_kernel(const uint8_t * 
 template <int EPI, bool FLAGGED>
 void launch_mx_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
     GemmArgs b = a;
-    b.row_units = static_cast<int>((rows + 127) / 128);
+    b.row_units = static_cast<int>((rows + 255) / 256);
     const int64_t items = static_cast<int64_t>(b.row_units) * max_tiles;
     hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)), dim3(kGemmThreads), 0,
                        stream, b);
@@ -1798,7 +1795,8 @@ void launch_grouped_gemm(const GemmParams & p, hipStream_t stream) {
     require(p.n_as >= 1 && p.n_as <= 1024 && p.n_entries >= 1, "GEMM group shape out of range");
     const int job_tile_n = gemm_job_tile(bank.type);
     const int64_t max_tiles = gemm_max_tiles(p.n_as, p.n_entries, job_tile_n);
-    require(max_tiles <= 65535, "too many GEMM tiles for one launch");
+    // the bound holds for tiles of 128 (MXFP4) and 192 (Q8_0) jobs, whatever tile the kernel takes
+    require(gemm_max_tiles(p.n_as, p.n_entries, bank.type == VBM_TYPE_MXFP4 ? 128 : 192) <= 65535, "too many GEMM tiles for one launch");
     int32_t * tile_expert = static_cast<int32_t *>(p.tiles);
     int32_t * tile_start = tile_expert + max_tiles;
     int32_t * n_tiles = tile_start + max_tiles;
