@@ -23,6 +23,8 @@
 // Epilogue 1 (fused gate|up bank): the workgroup's 64 rows are gate rows 32p..32p+31 and up rows
 // 32p..32p+31, i.e. exactly one 32-element Q8_0 block p of the GLU output; it applies the biases
 // and the GLU, requantizes (x86 contract) and writes the down projection's activation row.
+#include <type_traits>
+
 #include "vbm_device.hpp"
 #include "vbm_internal.hpp"
 
@@ -128,32 +130,15 @@ __device__ __forceinline__ Group load_group(const uint8_t * cp, const uint8_t * 
     return r;
 }
 
-// One MXFP4 block of one lane for MT tokens: bytes SEL, SEL+1 of `dw` are the slice's 4 nibbles;
-// the activation slice (4 f16 codes, 8 B per block) and the block scale of each token are read
-// from LDS (broadcast). Called by every lane of the wave (uniform control flow): the one- and
-// two-token form is a matrix-core instruction over the whole wave.
-template <int MT, bool SLOW, int SEL, int PAR>
+// The -128 path's blocks (caller-quantized rows holding such codes): the dots on the vector ALU, plus the
+// correction. One MXFP4 block of one lane for MT tokens: bytes SEL, SEL+1 of `dw` are the slice's 4
+// nibbles; the activation slice (4 f16 codes, 8 B per block) and the block scale of each token are read
+// from LDS (broadcast).
+template <int MT, int SEL, int PAR>
 __device__ __forceinline__ void mx_block(unsigned dw, int e, int b, const uint8_t * la, const float * lda,
                                          int tok_bytes, int mcount, float (&acc)[MT][2]) {
     const half2_t w01 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(dw, 2.0f, SEL);
     const half2_t w23 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(dw, 2.0f, SEL + 1);
-    if constexpr (MT <= 2 && !SLOW) {
-        // One v_mfma_f32_4x4x4_16b_f16 gives every token's slice dot: the row slice is B (lane =
-        // row) and lane 4q + r holds token r's activation slice as A, so register m of lane l is
-        // token m's dot with row l (exact: integers below 2^24), as in the single-token decode.
-        const int am = (threadIdx.x & 3) < mcount ? (threadIdx.x & 3) : 0;
-        const u32x2 a = *reinterpret_cast<const u32x2 *>(la + am * tok_bytes + b * 8);
-        const f32x4_t v = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, a), half4_t{w01.x, w01.y, w23.x, w23.y},
-                                                             f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m < mcount) {
-                const float d = *reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(lda) + m * tok_bytes + b * 4);
-                acc[m][PAR] = __builtin_fmaf(__builtin_amdgcn_ldexpf(d, e), v[m], acc[m][PAR]);
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         if (m < mcount) {
@@ -161,7 +146,7 @@ __device__ __forceinline__ void mx_block(unsigned dw, int e, int b, const uint8_
             const float d = *reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(lda) + m * tok_bytes + b * 4);
             float v = __builtin_amdgcn_fdot2(w23, as_half2(a.y), 0.0f, false);
             v = __builtin_amdgcn_fdot2(w01, as_half2(a.x), v, false);
-            if (SLOW) v += neg128_fix_half(w01, w23, a.x, a.y);
+            v += neg128_fix_half(w01, w23, a.x, a.y);
             const float s = __builtin_amdgcn_ldexpf(d, e);
             acc[m][PAR] = __builtin_fmaf(s, v, acc[m][PAR]);
         }
@@ -169,21 +154,21 @@ __device__ __forceinline__ void mx_block(unsigned dw, int e, int b, const uint8_
 }
 
 // Eight MXFP4 blocks (one group, starting at block b) for MT tokens.
-template <int MT, bool SLOW>
+template <int MT>
 __device__ __forceinline__ void mx_group(const u32x4 & c, const u32x2 & m, int b, const uint8_t * la, const float * lda,
                                          int tok_bytes, int mcount, float (&acc)[MT][2]) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const unsigned dw = q == 0 ? c.x : (q == 1 ? c.y : (q == 2 ? c.z : c.w));
         const unsigned ew = q < 2 ? m.x : m.y;
-        mx_block<MT, SLOW, 0, 0>(dw, static_cast<signed char>(ew >> ((2 * q & 3) * 8)), b + 2 * q, la, lda, tok_bytes,
+        mx_block<MT, 0, 0>(dw, static_cast<signed char>(ew >> ((2 * q & 3) * 8)), b + 2 * q, la, lda, tok_bytes,
                                  mcount, acc);
-        mx_block<MT, SLOW, 2, 1>(dw, static_cast<signed char>(ew >> (((2 * q + 1) & 3) * 8)), b + 2 * q + 1, la, lda,
+        mx_block<MT, 2, 1>(dw, static_cast<signed char>(ew >> (((2 * q + 1) & 3) * 8)), b + 2 * q + 1, la, lda,
                                  tok_bytes, mcount, acc);
     }
 }
 
-template <int MT, bool SLOW>
+template <int MT>
 __device__ __forceinline__ void q8_block(unsigned w, unsigned short dbits, int b, const uint8_t * la, const float * lda,
                                          int tok_bytes, int mcount, float (&acc)[MT][2]) {
     const float dw = half_bits_to_float(dbits);
@@ -193,7 +178,7 @@ __device__ __forceinline__ void q8_block(unsigned w, unsigned short dbits, int b
             const unsigned a = *reinterpret_cast<const unsigned *>(la + m * tok_bytes + b * 4);
             const float d = *reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(lda) + m * tok_bytes + b * 4);
             int v = __builtin_amdgcn_sdot4(static_cast<int>(w), static_cast<int>(a), 0, false);
-            if (SLOW) v += neg128_fix_i8(w, a);
+            v += neg128_fix_i8(w, a);
             const float s = dw * d;
             acc[m][0] = __builtin_fmaf(s, static_cast<float>(v), acc[m][0]);
         }
@@ -201,13 +186,13 @@ __device__ __forceinline__ void q8_block(unsigned w, unsigned short dbits, int b
 }
 
 // Four Q8_0 blocks (one group, starting at block b) for MT tokens: one chain per lane.
-template <int MT, bool SLOW>
+template <int MT>
 __device__ __forceinline__ void q8_group(const u32x4 & c, const u32x2 & m, int b, const uint8_t * la, const float * lda,
                                          int tok_bytes, int mcount, float (&acc)[MT][2]) {
-    q8_block<MT, SLOW>(c.x, static_cast<unsigned short>(m.x), b, la, lda, tok_bytes, mcount, acc);
-    q8_block<MT, SLOW>(c.y, static_cast<unsigned short>(m.x >> 16), b + 1, la, lda, tok_bytes, mcount, acc);
-    q8_block<MT, SLOW>(c.z, static_cast<unsigned short>(m.y), b + 2, la, lda, tok_bytes, mcount, acc);
-    q8_block<MT, SLOW>(c.w, static_cast<unsigned short>(m.y >> 16), b + 3, la, lda, tok_bytes, mcount, acc);
+    q8_block<MT>(c.x, static_cast<unsigned short>(m.x), b, la, lda, tok_bytes, mcount, acc);
+    q8_block<MT>(c.y, static_cast<unsigned short>(m.x >> 16), b + 1, la, lda, tok_bytes, mcount, acc);
+    q8_block<MT>(c.z, static_cast<unsigned short>(m.y), b + 2, la, lda, tok_bytes, mcount, acc);
+    q8_block<MT>(c.w, static_cast<unsigned short>(m.y >> 16), b + 3, la, lda, tok_bytes, mcount, acc);
 }
 
 // Weight groups a lane keeps in flight. Both MXFP4 decode kernels stream through a 5-deep ring
@@ -267,24 +252,22 @@ __device__ __forceinline__ void preload_ring(Group (&ring)[D], const uint8_t * c
 }
 
 // The tail blocks of one lane's row slice (after its full groups: block order is chain order).
-// With MLDS the exponents / scales come from the lane's tile meta staged in LDS (`meta_lds`).
-template <int TYPE, int MT, bool SLOW, bool MLDS>
-__device__ __forceinline__ void apply_tail(const Tail & tl, const uint8_t * meta_lds, int r, int nb, const uint8_t * la,
-                                           const float * lda, int tok_bytes, int mcount, float (&acc)[MT][2]) {
-    constexpr int kGroupBlocks = TYPE == 39 ? 8 : 4, kMeta = TYPE == 39 ? 1 : 2;
+template <int TYPE, int MT>
+__device__ __forceinline__ void apply_tail(const Tail & tl, int nb, const uint8_t * la, const float * lda,
+                                           int tok_bytes, int mcount, float (&acc)[MT][2]) {
+    constexpr int kGroupBlocks = TYPE == 39 ? 8 : 4;
     const int groups = nb / kGroupBlocks, tail = nb % kGroupBlocks;
     const int n = TYPE == 39 ? tail / 2 : tail;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         if (i < n) {
-            const unsigned m = MLDS ? *reinterpret_cast<const unsigned short *>(meta_lds + groups * 256 + r * tail * kMeta + 2 * i)
-                                    : tl.m[i];
+            const unsigned m = tl.m[i];
             if (TYPE == 39) {
                 const int b = groups * 8 + 2 * i;
-                mx_block<MT, SLOW, 0, 0>(tl.c[i], static_cast<signed char>(m & 0xFFu), b, la, lda, tok_bytes, mcount, acc);
-                mx_block<MT, SLOW, 2, 1>(tl.c[i], static_cast<signed char>(m >> 8), b + 1, la, lda, tok_bytes, mcount, acc);
+                mx_block<MT, 0, 0>(tl.c[i], static_cast<signed char>(m & 0xFFu), b, la, lda, tok_bytes, mcount, acc);
+                mx_block<MT, 2, 1>(tl.c[i], static_cast<signed char>(m >> 8), b + 1, la, lda, tok_bytes, mcount, acc);
             } else {
-                q8_block<MT, SLOW>(tl.c[i], static_cast<unsigned short>(m), groups * 4 + i, la, lda, tok_bytes, mcount, acc);
+                q8_block<MT>(tl.c[i], static_cast<unsigned short>(m), groups * 4 + i, la, lda, tok_bytes, mcount, acc);
             }
         }
     }
@@ -359,7 +342,7 @@ __device__ __forceinline__ void preload_tail_buf(Tail & t, const BufLane & B, in
     }
 }
 
-template <int TYPE, int MT, bool SLOW, int D>
+template <int TYPE, int MT, int D>
 __device__ __forceinline__ void stream_groups_buf(Group (&ring)[D], const BufLane & B, int nb, const uint8_t * la,
                                                   const float * lda, int tok_bytes, int mcount, float (&acc)[MT][2]) {
     constexpr int kGroupBlocks = TYPE == 39 ? 8 : 4;
@@ -371,100 +354,143 @@ __device__ __forceinline__ void stream_groups_buf(Group (&ring)[D], const BufLan
             if (g < groups) {
                 const Group cur = ring[i];
                 if (g + D < groups) ring[i] = load_group_buf(B, g + D);
-                if (TYPE == 39) mx_group<MT, SLOW>(cur.c, cur.m, g * 8, la, lda, tok_bytes, mcount, acc);
-                else q8_group<MT, SLOW>(cur.c, cur.m, g * 4, la, lda, tok_bytes, mcount, acc);
+                if (TYPE == 39) mx_group<MT>(cur.c, cur.m, g * 8, la, lda, tok_bytes, mcount, acc);
+                else q8_group<MT>(cur.c, cur.m, g * 4, la, lda, tok_bytes, mcount, acc);
             }
         }
     }
 }
 
-// ------------------------------------------------------ batched MXFP4 GEMV on the matrix cores
-// Chunks of four or more tokens without the -128 correction take the lane slices' integer dots
-// from v_mfma_f32_4x4x4_16b_f16, whose output register r of lane l is the dot over k of
-// A(lane 4(l/4) + r, k) and B(lane l, k). A is the lane's own row slice (lane = row, as in the
-// scalar path) and B the activation slice of token 4g + l % 4, so register r of lane l holds the
-// slice dot of row 4(l/4) + r and token 4g + l % 4: one instruction gives the wave's 64 rows x 4
-// tokens, each the value the two v_dot2 of the scalar path give (integers below 2^24 are exact
-// in any order). Every (row, token, slice) keeps the CPU's chains: one FMA per block into the even
-// or odd chain of the block.
+// ------------------------------------------------------------ batched GEMV on the matrix cores
+// Without the -128 correction the lane slices' integer dots come from v_mfma_f32_4x4x4_16b_f16 (MXFP4)
+// or v_mfma_i32_4x4x4_16b_i8 (Q8_0): 16 blocks of 4 x 4 outputs with K = 4, exactly one slice. B is the
+// lane's own row slice (lane = row, as in the scalar path). A is four tokens' activation slices of one
+// quantization block, broadcast from one of the instruction's 16 blocks to all of them (CBSZ = 4, ABID =
+// the block), so register m of lane l is the slice dot of row l and token m: exact (integers below 2^24,
+// or int32). One 8-byte (4-byte) LDS read per lane thus brings 16 quantization blocks of four tokens, and
+// one 4-byte read 16 block scales of a token, which the sums take through a row broadcast (DPP), where a
+// read of codes and of scales per block and lane returned 768 bytes for one MFMA and four FMAs. Activations
+// stay staged in LDS: read from their rows in global memory instead, 32 tokens over 128 experts took 286
+// against 217 us, and 16-token chunks, for which LDS has no room, gained nothing. Registers are held to 80
+// (six waves per SIMD, three workgroups per CU): at 88 the same code took 643 against 538 us for 256 tokens
+// (top-4 over 32 experts, hidden = inter = 2880).
+// Every (row, token, slice) keeps the CPU's chains: one FMA per block into the even or odd chain of
+// the block (one chain for Q8_0).
 //
-// FOLD: when every exponent e of the tile pair's rows lies in [-14, 12], the conversion
+// FOLD (MXFP4): when every exponent e of the tile pair's rows lies in [-14, 12], the conversion
 // scales the e2m1 values by 2^(e+1) (exact normal f16), the dot comes out as 2^e * dot, and the
 // chain's FMA takes d_act alone: d_act * (2^e * dot) is exactly the product ldexp(d_act, e) * dot
-// (no overflow or underflow in that range), rounded once inside the same FMA. Otherwise each
-// output takes ldexp(d_act, e) with e broadcast from its row's lane within the quad.
-template <int MT>
-using MmAcc = float[MT / 4][4][2];
+// (no overflow or underflow in that range), rounded once inside the same FMA.
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
-// One block for the MT / 4 token groups: `a[g]` is token group g's activation slice (4 f16 codes)
-// and `d[g]` its block scale, both for the lane's token 4g + l % 4.
-template <int MT, int SEL, int PAR, bool FOLD>
-__device__ __forceinline__ void mx_block_mm(unsigned dw, int e, const u32x2 (&a)[MT / 4], const float (&d)[MT / 4],
-                                            MmAcc<MT> & acc) {
-    constexpr int G = MT / 4;
-    const float sc = FOLD ? __builtin_bit_cast(float, (e + 128) << 23) : 2.0f;
-    const half2_t w01 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(dw, sc, SEL);
-    const half2_t w23 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(dw, sc, SEL + 1);
-    const half4_t wv = half4_t{w01.x, w01.y, w23.x, w23.y};
-    f32x4_t v[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-        v[g] = __builtin_amdgcn_mfma_f32_4x4x4f16(wv, __builtin_bit_cast(half4_t, a[g]), f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-    if constexpr (FOLD) {
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[g][r][PAR] = __builtin_fmaf(d[g], v[g][r], acc[g][r][PAR]);
-    } else {
-        int eq[4];
-        eq[0] = __builtin_amdgcn_mov_dpp(e, 0x00, 0xf, 0xf, false);   // quad_perm [r, r, r, r]
-        eq[1] = __builtin_amdgcn_mov_dpp(e, 0x55, 0xf, 0xf, false);
-        eq[2] = __builtin_amdgcn_mov_dpp(e, 0xAA, 0xf, 0xf, false);
-        eq[3] = __builtin_amdgcn_mov_dpp(e, 0xFF, 0xf, 0xf, false);
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                acc[g][r][PAR] = __builtin_fmaf(__builtin_amdgcn_ldexpf(d[g], eq[r]), v[g][r], acc[g][r][PAR]);
-    }
+// Lane n of each row of 16 lanes, in every lane of the row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + N, 0xF, 0xF, true));
 }
 
-// Two consecutive blocks b, b + 1 of one code dword (e0, e1 their exponents); `a2[g]` holds both
-// blocks' activation slices of token group g, `d0[g]` / `d1[g]` their scales.
-template <int MT, bool FOLD>
-__device__ __forceinline__ void mx_pair_mm(unsigned dw, int e0, int e1, const u32x4 (&a2)[MT / 4], const float (&d0)[MT / 4],
-                                           const float (&d1)[MT / 4], MmAcc<MT> & acc) {
-    constexpr int G = MT / 4;
-    u32x2 a0[G], a1[G];
+// acc[m][PAR] = fma(row_bcast<N>(d[m]), v[m], acc[m][PAR]) for every token. The compiler does not fold a row
+// broadcast into an FMA (a move per token otherwise, as many as the FMAs), so the instructions are written
+// out. The s_nop ahead of them stands in for the wait states the compiler gives its own instructions: five
+// between a two-pass MFMA and a read of its result, two between a VALU write and a DPP read of it.
+#define VBM_FMAC_BCAST(acc, d, v) "v_fmac_f32_dpp %" #acc ", %" #d ", %" #v " row_newbcast:%c[n] row_mask:0xf bank_mask:0xf\n\t"
+template <int M, int PAR, int N>
+__device__ __forceinline__ void fma_bcast(float (&acc)[M][2], const float (&d)[M], const f32x4_t (&v)[(M + 3) / 4]) {
+    if constexpr (M == 1)
+        asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 1, 2) : "+v"(acc[0][PAR]) : "v"(d[0]), "v"(v[0][0]), [n] "n"(N));
+    else if constexpr (M == 2)
+        asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 2, 4) VBM_FMAC_BCAST(1, 3, 5)
+            : "+v"(acc[0][PAR]), "+v"(acc[1][PAR]) : "v"(d[0]), "v"(d[1]), "v"(v[0][0]), "v"(v[0][1]), [n] "n"(N));
+    else {
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        a0[g] = u32x2{a2[g].x, a2[g].y};
-        a1[g] = u32x2{a2[g].z, a2[g].w};
+        for (int g = 0; g < M / 4; ++g)
+            asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 4, 8) VBM_FMAC_BCAST(1, 5, 9) VBM_FMAC_BCAST(2, 6, 10) VBM_FMAC_BCAST(3, 7, 11)
+                : "+v"(acc[4 * g][PAR]), "+v"(acc[4 * g + 1][PAR]), "+v"(acc[4 * g + 2][PAR]), "+v"(acc[4 * g + 3][PAR])
+                : "v"(d[4 * g]), "v"(d[4 * g + 1]), "v"(d[4 * g + 2]), "v"(d[4 * g + 3]), "v"(v[g][0]), "v"(v[g][1]), "v"(v[g][2]),
+                  "v"(v[g][3]), [n] "n"(N));
     }
-    mx_block_mm<MT, 0, 0, FOLD>(dw, e0, a0, d0, acc);
-    mx_block_mm<MT, 2, 1, FOLD>(dw, e1, a1, d1, acc);
 }
+#undef VBM_FMAC_BCAST
 
-// One group of eight blocks starting at block b; each block reads its activation slices and
-// scales itself, and the fence after it keeps the scheduler from hoisting every read of the group
-// (register spills otherwise).
-template <int MT, bool FOLD>
-__device__ __forceinline__ void mx_group_mm(const u32x4 & c, const u32x2 & m, int b, const uint8_t * la_lane,
-                                            const uint8_t * lda_lane, int tok_bytes, MmAcc<MT> & acc) {
-    constexpr int G = MT / 4;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const unsigned dw = c[j >> 1];
-        const int e = static_cast<signed char>((j < 4 ? m.x : m.y) >> (8 * (j & 3)));
-        u32x2 a[G];
-        float d[G];
+// Activations of 16 quantization blocks from b0: lane 4n + i holds the wave's slice of block b0 + n of token
+// 4g + i in a[g]; lane n of each 16-lane row holds the scale of block b0 + n of token m in d[m].
+template <int TYPE, int M>
+struct ActBlocks {
+    static constexpr int G = (M + 3) / 4;
+    u32x2 a[G];
+    float d[M];
+    __device__ __forceinline__ void load(const uint8_t * la, const uint8_t * lda, int tok_bytes, int b0, int nb) {
+        const int lane = threadIdx.x & 63;
+        const int ba = b0 + (lane >> 2) < nb ? b0 + (lane >> 2) : nb - 1, bd = b0 + (lane & 15) < nb ? b0 + (lane & 15) : nb - 1;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            a[g] = *reinterpret_cast<const u32x2 *>(la_lane + 4 * g * tok_bytes + (b + j) * 8);
-            d[g] = *reinterpret_cast<const float *>(lda_lane + 4 * g * tok_bytes + (b + j) * 4);
+            const int t = M < 4 && (lane & 3) >= M ? 0 : 4 * g + (lane & 3);
+            if (TYPE == 39) a[g] = *reinterpret_cast<const u32x2 *>(la + t * tok_bytes + ba * 8);
+            else a[g].x = *reinterpret_cast<const unsigned *>(la + t * tok_bytes + ba * 4);
         }
-        if (j & 1) mx_block_mm<MT, 2, 1, FOLD>(dw, e, a, d, acc);
-        else mx_block_mm<MT, 0, 0, FOLD>(dw, e, a, d, acc);
+#pragma unroll
+        for (int m = 0; m < M; ++m) d[m] = *reinterpret_cast<const float *>(lda + m * tok_bytes + bd * 4);
+    }
+};
+
+// Block N of the 16 in `act`. MXFP4: bytes SEL, SEL + 1 of `w` are the slice's nibbles, `raw` its e8m0
+// exponent byte + 1 in the low byte of a word shifted into the f32 exponent field by the caller (FOLD) or the
+// signed exponent; Q8_0: `w` the four codes, dw the block's scale.
+template <int M, int SEL, int PAR, int N, bool FOLD>
+__device__ __forceinline__ void mx_block_mm(unsigned w, float fold_scale, int e, const ActBlocks<39, M> & act, float (&acc)[M][2]) {
+    const float sc = FOLD ? fold_scale : 2.0f;
+    const half2_t w01 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, SEL);
+    const half2_t w23 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, sc, SEL + 1);
+    const half4_t wv = half4_t{w01.x, w01.y, w23.x, w23.y};
+    f32x4_t v[ActBlocks<39, M>::G];
+#pragma unroll
+    for (int g = 0; g < ActBlocks<39, M>::G; ++g)
+        v[g] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, act.a[g]), wv, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 4, N, 0);
+    if constexpr (FOLD) {
+        fma_bcast<M, PAR, N>(acc, act.d, v);
+    } else {
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            acc[m][PAR] = __builtin_fmaf(__builtin_amdgcn_ldexpf(row_bcast<N>(act.d[m]), e), v[m / 4][m % 4], acc[m][PAR]);
+    }
+}
+template <int M, int N>
+__device__ __forceinline__ void q8_block_mm(unsigned w, float dw, const ActBlocks<8, M> & act, float (&acc)[M][2]) {
+    i32x4_t v[ActBlocks<8, M>::G];
+#pragma unroll
+    for (int g = 0; g < ActBlocks<8, M>::G; ++g)
+        v[g] = __builtin_amdgcn_mfma_i32_4x4x4i8(static_cast<int>(act.a[g].x), static_cast<int>(w), i32x4_t{0, 0, 0, 0}, 4, N, 0);
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+        acc[m][0] = __builtin_fmaf(dw * row_bcast<N>(act.d[m]), static_cast<float>(v[m / 4][m % 4]), acc[m][0]);
+}
+
+// One bank group whose first block is block N0 of the 16 in `act` (the fence after each pair of blocks keeps
+// the scheduler from converting the whole group ahead).
+template <int TYPE, int M, int N0, bool FOLD>
+__device__ __forceinline__ void group_mm(const u32x4 & c, const u32x2 & m, const ActBlocks<TYPE, M> & act, float (&acc)[M][2]) {
+    if constexpr (TYPE == 39) {
+        const unsigned r0 = m.x ^ 0x80808080u, r1 = m.y ^ 0x80808080u;   // raw e8m0 bytes: 2^(e+1) is byte << 23
+        auto pair = [&](auto q_c) __attribute__((always_inline)) {
+            constexpr int Q = decltype(q_c)::value;
+            const unsigned r = Q < 2 ? r0 : r1, s = Q < 2 ? m.x : m.y;
+            constexpr int B0 = 16 * (Q & 1), B1 = B0 + 8;
+            mx_block_mm<M, 0, 0, N0 + 2 * Q, FOLD>(c[Q], __builtin_bit_cast(float, ((r >> B0) & 0xFFu) << 23),
+                                                   static_cast<signed char>(s >> B0), act, acc);
+            mx_block_mm<M, 2, 1, N0 + 2 * Q + 1, FOLD>(c[Q], __builtin_bit_cast(float, ((r >> B1) & 0xFFu) << 23),
+                                                       static_cast<signed char>(s >> B1), act, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        pair(std::integral_constant<int, 0>{});
+        pair(std::integral_constant<int, 1>{});
+        pair(std::integral_constant<int, 2>{});
+        pair(std::integral_constant<int, 3>{});
+    } else {
+        q8_block_mm<M, N0>(c.x, half_bits_to_float(static_cast<uint16_t>(m.x)), act, acc);
+        q8_block_mm<M, N0 + 1>(c.y, half_bits_to_float(static_cast<uint16_t>(m.x >> 16)), act, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        q8_block_mm<M, N0 + 2>(c.z, half_bits_to_float(static_cast<uint16_t>(m.y)), act, acc);
+        q8_block_mm<M, N0 + 3>(c.w, half_bits_to_float(static_cast<uint16_t>(m.y >> 16)), act, acc);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -480,53 +506,58 @@ __device__ __forceinline__ bool exps_foldable(const u32x4 & w) {
     return ok;
 }
 
-template <int MT, int D, bool FOLD>
-__device__ __forceinline__ void stream_groups_mm(Group (&ring)[D], const BufLane & B, int nb, const uint8_t * la_lane,
-                                                 const uint8_t * lda_lane, int tok_bytes, MmAcc<MT> & acc) {
-    const int groups = nb / 8;
-    for (int g0 = 0; g0 < groups; g0 += D) {
-#pragma unroll
-        for (int i = 0; i < D; ++i) {
-            const int g = g0 + i;
-            if (g < groups) {
-                const Group cur = ring[i];
-                if (g + D < groups) ring[i] = load_group_buf(B, g + D);
-                mx_group_mm<MT, FOLD>(cur.c, cur.m, g * 8, la_lane, lda_lane, tok_bytes, acc);
+// Every full group of one lane's row slice, 16 blocks (2 MXFP4 or 4 Q8_0 groups) per activation load.
+template <int TYPE, int M, int D, bool FOLD>
+__device__ __forceinline__ void stream_groups_mm(Group (&ring)[D], const BufLane & B, int nb, const uint8_t * la,
+                                                 const uint8_t * lda, int tok_bytes, float (&acc)[M][2]) {
+    constexpr int GB = TYPE == 39 ? 8 : 4, U = 16 / GB;
+    static_assert(U % D == 0, "the ring index is the group's place in the 16 blocks");
+    const int groups = nb / GB;
+#pragma clang loop unroll(disable)
+    for (int g0 = 0; g0 < groups; g0 += U) {
+        ActBlocks<TYPE, M> act;
+        act.load(la, lda, tok_bytes, g0 * GB, nb);
+        auto step = [&](auto i_c) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_c)::value;
+            if constexpr (i < U) {
+                const int g = g0 + i;
+                if (g < groups) {
+                    const Group cur = ring[i % D];
+                    if (g + D < groups) ring[i % D] = load_group_buf(B, g + D);
+                    group_mm<TYPE, M, GB * i, FOLD>(cur.c, cur.m, act, acc);
+                }
             }
-        }
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
     }
 }
 
 // The tail blocks (after the full groups, in chain order) with the unfolded scales.
-template <int MT>
-__device__ __forceinline__ void apply_tail_mm(const Tail & tl, int nb, const uint8_t * la_lane, const uint8_t * lda_lane,
-                                              int tok_bytes, MmAcc<MT> & acc) {
-    constexpr int G = MT / 4;
-    const int groups = nb / 8, n = (nb % 8) / 2;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
+template <int TYPE, int M>
+__device__ __forceinline__ void apply_tail_mm(const Tail & tl, int nb, const uint8_t * la, const uint8_t * lda, int tok_bytes,
+                                              float (&acc)[M][2]) {
+    constexpr int GB = TYPE == 39 ? 8 : 4;
+    const int b0 = nb / GB * GB, n = TYPE == 39 ? (nb - b0) / 2 : nb - b0;
+    if (n == 0) return;
+    ActBlocks<TYPE, M> act;
+    act.load(la, lda, tok_bytes, b0, nb);
+    auto step = [&](auto i_c) __attribute__((always_inline)) {
+        constexpr int i = decltype(i_c)::value;
         if (i < n) {
-            const int b = groups * 8 + 2 * i;
-            u32x4 a2[G];
-            float d0[G], d1[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                a2[g] = *reinterpret_cast<const u32x4 *>(la_lane + 4 * g * tok_bytes + b * 8);
-                const float * dp = reinterpret_cast<const float *>(lda_lane + 4 * g * tok_bytes + b * 4);
-                d0[g] = dp[0];
-                d1[g] = dp[1];
+            if constexpr (TYPE == 39) {
+                mx_block_mm<M, 0, 0, 2 * i, false>(tl.c[i], 0.0f, static_cast<signed char>(tl.m[i] & 0xFFu), act, acc);
+                mx_block_mm<M, 2, 1, 2 * i + 1, false>(tl.c[i], 0.0f, static_cast<signed char>(tl.m[i] >> 8), act, acc);
+            } else {
+                q8_block_mm<M, i>(tl.c[i], half_bits_to_float(static_cast<uint16_t>(tl.m[i])), act, acc);
             }
-            mx_pair_mm<MT, false>(tl.c[i], static_cast<signed char>(tl.m[i] & 0xFFu), static_cast<signed char>(tl.m[i] >> 8),
-                                  a2, d0, d1, acc);
         }
-    }
-}
-
-// The matrix-core path serves MXFP4 chunks of four or more tokens in the kernels for rows this
-// library quantized (never -128); the kernels for caller-quantized rows keep the scalar path.
-template <int TYPE, int M, bool NEG>
-constexpr bool use_mfma() {
-    return TYPE == 39 && M >= 4 && !NEG;
+    };
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
 }
 
 // Stages the exponents / scales of a workgroup's (up to) two consecutive tiles: loads are issued
@@ -774,9 +805,9 @@ __device__ __forceinline__ void glu_requant_block(const float * vals, int lane, 
 // stream every lane's row slice once applying each token, reduce the eight slices per token and
 // write the outputs (or the GLU block). M is the narrowest token width holding the chunk.
 template <int TYPE, int M, bool NEG>
-__device__ __forceinline__ void gemv_chunk(const KernelArgs & A, const BufLane & B, const __attribute__((address_space(4))) int32_t * jobs,
+__device__ __forceinline__ void gemv_chunk(const KernelArgs & A, const BufLane & B, const int32_t * jobs_v,
                                            int expert, int c0, int mcount, int pair, int k, int lane, int r, int tile,
-                                           bool live, uint8_t * lds_tok, float * red, float * vals, int * s_flag) {
+                                           bool live, uint8_t * lds_tok, float * red, float * vals) {
     const Shape S = A.shape;
     const int nb = S.nb;
     const int copy_bytes = static_cast<int>(A.lay.flag_offset());        // codes + scales of a row
@@ -796,77 +827,65 @@ __device__ __forceinline__ void gemv_chunk(const KernelArgs & A, const BufLane &
     // the tile pair's live rows lies in [-14, 12]: one 16-byte load per thread (K <= 4096: at most
     // 8 KiB of exponents), issued with the ring and checked at the staging barrier.
     u32x4 ex = u32x4{0u, 0u, 0u, 0u};
-    if constexpr (use_mfma<TYPE, M, NEG>()) {
+    if constexpr (TYPE == 39) {
         const int pair_tiles = (2 * pair + 1) * 32 < S.rows ? 2 : 1;
         const int meta0 = static_cast<int>(S.codes_bytes) + 2 * pair * 32 * nb;
         if (static_cast<int>(threadIdx.x) * 16 < pair_tiles * 32 * nb)
             ex = __builtin_amdgcn_raw_buffer_load_b128(B.rsrc, meta0 + static_cast<int>(threadIdx.x) * 16, 0, 0);
     }
-    // Stage the chunk's activation rows (and their -128 flags) in LDS.
-    if (threadIdx.x == 0) *s_flag = 0;
-    __syncthreads();
-    int flag = 0;
-    for (int mi = 0; mi < mcount; ++mi) {
-        const int64_t j = jobs[c0 + mi];
-        const int64_t row = A.b_ne1 == 1 ? j / A.n_ids : j;
-        const uint8_t * xr = A.xrows + row * A.lay.stride();
-        uint8_t * dst = lds_tok + mi * tok_bytes;
-        for (int i = threadIdx.x; i * 16 < copy_bytes - 15; i += kThreads)
-            *reinterpret_cast<u32x4 *>(dst + i * 16) = *reinterpret_cast<const u32x4 *>(xr + i * 16);
-        for (int i = (copy_bytes & ~15) + threadIdx.x * 4; i < copy_bytes; i += kThreads * 4)
-            *reinterpret_cast<unsigned *>(dst + i) = *reinterpret_cast<const unsigned *>(xr + i);
-        if (threadIdx.x == 0) flag |= *reinterpret_cast<const int *>(xr + A.lay.flag_offset());
+    // Lane t: job and activation row of token t (past the chunk: token 0's).
+    const uint32_t job = static_cast<uint32_t>(jobs_v[c0 + (lane < mcount ? lane : 0)]);
+    const uint32_t row = A.b_ne1 == 1 ? job / static_cast<uint32_t>(A.n_ids) : job;
+    const int grow = static_cast<int>(ggml_row(static_cast<int64_t>(live ? tile : 0) * 32 + r, S.rows, S.interleave));
+    const float bias_v = A.bias ? A.bias[static_cast<size_t>(expert) * S.rows + grow] : 0.0f;
+    // Stage the chunk's activation rows in LDS, 16 bytes per thread and token with every token's load in
+    // flight together (one token after another cost a memory latency each: 538 against 462 us for the 256
+    // tokens above, 193 against 164 us for 64). The last piece reads past the scales into the row's own
+    // padding.
+    for (int i = threadIdx.x; i * 16 < tok_bytes; i += kThreads) {
+        u32x4 v[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            v[m] = *reinterpret_cast<const u32x4 *>(A.xrows + static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(row), m))) *
+                                                                  static_cast<uint64_t>(A.lay.stride()) + i * 16);
+#pragma unroll
+        for (int m = 0; m < M; ++m) *reinterpret_cast<u32x4 *>(lds_tok + m * tok_bytes + i * 16) = v[m];
     }
-    if (threadIdx.x == 0 && flag) *s_flag = 1;
+    bool slow = false;
+    if constexpr (NEG) {
+        int flag = 0;
+        if (lane < mcount) flag = *reinterpret_cast<const int *>(A.xrows + static_cast<uint64_t>(row) * static_cast<uint64_t>(A.lay.stride()) + A.lay.flag_offset());
+        slow = __any(flag != 0);                             // every wave reads the same flags: workgroup-uniform
+    }
     bool fold = false;
-    if constexpr (use_mfma<TYPE, M, NEG>()) fold = __syncthreads_and(exps_foldable(ex) ? 1 : 0) != 0;
+    if constexpr (TYPE == 39) fold = __syncthreads_and(exps_foldable(ex) ? 1 : 0) != 0;
     else __syncthreads();
     Tail tl;
-    if constexpr (use_mfma<TYPE, M, NEG>()) {
-        MmAcc<M> acc;
+    float acc[M][2];
 #pragma unroll
-        for (int g = 0; g < M / 4; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[g][i][0] = acc[g][i][1] = 0.0f;
-        const uint8_t * la_lane = la + (lane & 3) * tok_bytes;   // token 4g + lane % 4
-        const uint8_t * lda_lane = reinterpret_cast<const uint8_t *>(lda) + (lane & 3) * tok_bytes;
-        if (fold) stream_groups_mm<M, D, true>(ring, B, nb, la_lane, lda_lane, tok_bytes, acc);
-        else stream_groups_mm<M, D, false>(ring, B, nb, la_lane, lda_lane, tok_bytes, acc);
-        preload_tail_buf<TYPE>(tl, B, nb);
-        apply_tail_mm<M>(tl, nb, la_lane, lda_lane, tok_bytes, acc);
-        __syncthreads();   // `red` reuses the staged activation rows the other waves may still read
-        // register i of lane l: row 4(l / 4) + i (the red layout's lane index) of token 4g + l % 4
-#pragma unroll
-        for (int g = 0; g < M / 4; ++g)
-            *reinterpret_cast<float4 *>(&red[((4 * g + (lane & 3)) * 8 + k) * 64 + 4 * (lane >> 2)]) =
-                float4{acc[g][0][0] + acc[g][0][1], acc[g][1][0] + acc[g][1][1], acc[g][2][0] + acc[g][2][1],
-                       acc[g][3][0] + acc[g][3][1]};
-    } else {
-        float acc[M][2];
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[m][0] = acc[m][1] = 0.0f;
-        // widths 1 and 2 only ever carry full chunks: a constant count drops the per-token checks
-        const int mc = M <= 2 ? M : mcount;
-        if (NEG && *s_flag) {
-            stream_groups_buf<TYPE, M, true, D>(ring, B, nb, la, lda, tok_bytes, mc, acc);
+    for (int m = 0; m < M; ++m) acc[m][0] = acc[m][1] = 0.0f;
+    if (NEG && slow) {
+        if constexpr (NEG) {
+            stream_groups_buf<TYPE, M, D>(ring, B, nb, la, lda, tok_bytes, mcount, acc);
             preload_tail_buf<TYPE>(tl, B, nb);
-            apply_tail<TYPE, M, true, false>(tl, nullptr, r, nb, la, lda, tok_bytes, mc, acc);
-        } else {
-            stream_groups_buf<TYPE, M, false, D>(ring, B, nb, la, lda, tok_bytes, mc, acc);
-            preload_tail_buf<TYPE>(tl, B, nb);
-            apply_tail<TYPE, M, false, false>(tl, nullptr, r, nb, la, lda, tok_bytes, mc, acc);
+            apply_tail<TYPE, M>(tl, nb, la, lda, tok_bytes, mcount, acc);
         }
-        __syncthreads();   // `red` reuses the staged activation rows the other waves may still read
-#pragma unroll
-        for (int m = 0; m < M; ++m) red[(m * 8 + k) * 64 + lane] = acc[m][0] + acc[m][1];
+    } else {
+        const uint8_t * ldab = reinterpret_cast<const uint8_t *>(lda);
+        if (TYPE == 39 && !fold) stream_groups_mm<TYPE, M, D, false>(ring, B, nb, la, ldab, tok_bytes, acc);
+        else stream_groups_mm<TYPE, M, D, true>(ring, B, nb, la, ldab, tok_bytes, acc);
+        preload_tail_buf<TYPE>(tl, B, nb);
+        apply_tail_mm<TYPE, M>(tl, nb, la, ldab, tok_bytes, acc);
     }
+    __syncthreads();   // `red` reuses the staged activation rows the other waves may still read
+#pragma unroll
+    for (int m = 0; m < M; ++m) red[(m * 8 + k) * 64 + lane] = acc[m][0] + acc[m][1];
     __syncthreads();
     for (int mi = k; mi < mcount; mi += 8) {                           // wave k reduces tokens k, k+8, ...
         if (live) {
             float v = lane_tree(&red[mi * 8 * 64 + lane]);
-            const int grow = static_cast<int>(ggml_row(static_cast<int64_t>(tile) * 32 + r, S.rows, S.interleave));
-            if (A.bias) v = v + A.bias[static_cast<size_t>(expert) * S.rows + grow];
-            if (A.epilogue == 0) A.dst[static_cast<size_t>(jobs[c0 + mi]) * S.rows + grow] = v;
+            if (A.bias) v = v + bias_v;
+            if (A.epilogue == 0) A.dst[static_cast<size_t>(__builtin_amdgcn_readlane(static_cast<int>(job), mi)) * S.rows + grow] = v;
             else vals[mi * 64 + lane] = v;
         }
     }
@@ -874,10 +893,9 @@ __device__ __forceinline__ void gemv_chunk(const KernelArgs & A, const BufLane &
         __syncthreads();
         for (int mi = k; mi < mcount; mi += 8)
             if (lane < 32)
-                glu_requant_block(vals + mi * 64, lane, pair, A.dst_xrows + static_cast<size_t>(jobs[c0 + mi]) * A.dst_lay.stride(),
+                glu_requant_block(vals + mi * 64, lane, pair, A.dst_xrows + static_cast<size_t>(__builtin_amdgcn_readlane(static_cast<int>(job), mi)) * A.dst_lay.stride(),
                                   A.dst_lay, A.activation, A.alpha, A.limit);
     }
-    __syncthreads();
 }
 
 // Batched GEMV: one workgroup per (tile pair, chunk), a chunk being up to MT consecutive jobs of
@@ -890,9 +908,8 @@ __device__ __forceinline__ void gemv_chunk(const KernelArgs & A, const BufLane &
 // branch: most experts of a small decode batch see one or two tokens, and a narrow width keeps
 // the per-block token loop short).
 template <int TYPE, int MT, bool NEG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void expert_gemv_kernel(KernelArgs A) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6))) void expert_gemv_kernel(KernelArgs A) {
     __shared__ float vals[MT * 64];
-    __shared__ int s_flag;
     // MT activation rows; after the weight stream, the [MT][8 slices][64 rows] partial sums
     // (8 KiB less LDS per token of width than separate buffers: three workgroups per CU at MT = 8
     // with K = 2880)
@@ -910,7 +927,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int expert = as_const<int32_t>(A.chunk_expert)[item];
     const int c0 = as_const<int32_t>(A.chunk_start)[item];
     const int count = as_const<int32_t>(A.counts)[expert];
-    const __attribute__((address_space(4))) int32_t * jobs = as_const<int32_t>(A.rows_list) + as_const<int32_t>(A.offsets)[expert];
+    const int32_t * jobs_v = A.rows_list + as_const<int32_t>(A.offsets)[expert];
+    const __attribute__((address_space(4))) int32_t * jobs = as_const<int32_t>(jobs_v);
     const int slot = A.expert_to_slot ? as_const<int32_t>(A.expert_to_slot)[expert] : expert;
     const int mcount = count - c0 < MT ? count - c0 : MT;
     if (mcount <= 0) return;
@@ -942,13 +960,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const uint8_t * slot_base = A.bank + static_cast<size_t>(slot) * S.slot_bytes;
     const BufLane B = buf_lane<TYPE>(slot_base, S.slot_bytes, S.codes_bytes, live ? tile : 0, k, r, S.nb);
     if (MT >= 8 && mcount > 4)
-        gemv_chunk<TYPE, (MT >= 8 ? 8 : 1), NEG>(A, B, jobs, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals, &s_flag);
+        gemv_chunk<TYPE, (MT >= 8 ? 8 : 1), NEG>(A, B, jobs_v, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals);
     else if (MT >= 4 && mcount > 2)
-        gemv_chunk<TYPE, (MT >= 4 ? 4 : 1), NEG>(A, B, jobs, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals, &s_flag);
+        gemv_chunk<TYPE, (MT >= 4 ? 4 : 1), NEG>(A, B, jobs_v, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals);
     else if (MT >= 2 && mcount > 1)
-        gemv_chunk<TYPE, (MT >= 2 ? 2 : 1), NEG>(A, B, jobs, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals, &s_flag);
+        gemv_chunk<TYPE, (MT >= 2 ? 2 : 1), NEG>(A, B, jobs_v, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals);
     else
-        gemv_chunk<TYPE, 1, NEG>(A, B, jobs, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals, &s_flag);
+        gemv_chunk<TYPE, 1, NEG>(A, B, jobs_v, expert, c0, mcount, pair, k, lane, r, tile, live, lds_tok, red, vals);
 }
 
 // ------------------------------------------------------------------------------ fused decode
