@@ -1,0 +1,77 @@
+"""Sizes at which the kernels' tiles and dispatch rules change: MXFP4 prefill GEMM job tiles and row
+units, the router's two forms, and the one-token layer call."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import helpers as H
+from test_gpu_layer import Layer
+from test_gpu_prefill import unit_scale_activations, unit_scale_mxfp4, unit_scale_q8
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("type_id", [H.MX, H.Q8])
+@pytest.mark.parametrize("rows,k", [(288, 576), (544, 256)])
+def test_gemm_job_counts_around_the_tile_edges_exact(gpu, orc, type_id, rows, k):
+    """One expert per job count: 1, 15..17 and 63..65 jobs (fragment columns of 16, job tiles of 64), 130
+    jobs, and experts without any; rows past the 256-row units. Unit scales: every fp32 sum is an exact
+    integer, so any order gives the oracle's bits."""
+    counts = [1, 0, 15, 16, 17, 63, 64, 65, 130, 0, 33, 48, 96, 97]
+    ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
+    rng = np.random.default_rng(11 + rows)
+    rng.shuffle(ids)
+    ids = ids.reshape(-1, 1)
+    tokens = ids.shape[0]
+    w = (unit_scale_mxfp4 if type_id == H.MX else unit_scale_q8)(len(counts), rows, k, rng)
+    bank = H.make_bank(type_id, w, len(counts), rows, k)
+    x = unit_scale_activations(tokens, k, rng).reshape(tokens, 1, k)
+    got = H.mul_mat_id(bank, len(counts), x, gpu.TYPE_F32, 1, ids, 1, order=gpu.ORDER_FAST)
+    ref = orc.mul_mat_id(type_id, w, k, rows, len(counts), 0, x, 1, ids, 1, tokens, 1, threads=8)
+    assert H.bits_equal(got, ref), H.diff_report(got, ref)
+    bank.destroy()
+
+
+@pytest.mark.parametrize("n_expert,tokens,hidden", [(8, 3, 1000), (32, 1, 2880), (33, 250, 2880), (32, 257, 100), (64, 128, 960)])
+def test_router_logits_bitwise(gpu, orc, n_expert, tokens, hidden):
+    """One token per weight row and, from 8192 (expert, token) pairs on, four: ragged token counts, rows of
+    one batch of steps and of several, and rows with a remainder past the last 32 (summed serially)."""
+    w = gpu.synth_normal(15, 1, 0, n_expert * hidden, 0.0, 0.02).reshape(n_expert, hidden)
+    x = gpu.synth_normal(15, 2, 0, tokens * hidden).reshape(tokens, hidden)
+    dw, dx = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x)
+    dl, di, dwt = (gpu.DeviceBuffer(4 * tokens * n) for n in (n_expert, 2, 2))
+    gpu.call("vbm_router_topk_softmax", dw.ptr, None, dx.ptr, hidden, dl.ptr, n_expert, tokens, 2, di.ptr, dwt.ptr, None)
+    logits, ids, _ = orc.router(router_w=w, x=x, n_expert=n_expert, n_tokens=tokens, top_k=2, hidden=hidden)
+    assert H.bits_equal(dl.download(np.float32, (tokens, n_expert)), logits)
+    assert np.array_equal(di.download(np.int32, (tokens, 2)), ids)
+
+
+@pytest.mark.parametrize("type_id,hidden,inter,experts,top_k,act,biases", [
+    (H.MX, 2880, 2880, 32, 4, 1, True), (H.Q8, 2048, 768, 128, 8, 0, False), (H.MX, 64, 4096, 300, 3, 0, True),
+    (H.Q8, 4096, 64, 9, 9, 1, True), (H.MX, 448, 192, 5, 1, 1, False)])
+def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, experts, top_k, act, biases):
+    """A one-token call runs the decode kernels when its input is 16-byte aligned and the batched path
+    otherwise: the oracle's bits from both."""
+    layer = Layer(gpu, type_id, hidden, inter, experts, top_k, seed=91, router=False, biases=biases, activation=act,
+                  q8_scale=(1e-4, 1e-3))
+    x = gpu.synth_normal(91, 6, 0, hidden).reshape(1, hidden)
+    logits = gpu.synth_normal(91, 7, 0, experts).reshape(1, experts)
+    logits[0, : experts // 2] = np.round(logits[0, : experts // 2])          # ties
+    ref = layer.forward_cpu(orc, x, logits)
+    d = layer.desc()
+    need = C.c_size_t()
+    gpu.call("vbm_moe_layer_workspace", C.byref(d), 1, C.byref(need))
+    work = gpu.DeviceBuffer(need.value)
+    dx = gpu.DeviceBuffer.from_array(x)
+    off = gpu.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x[0]]))
+    dl = gpu.DeviceBuffer.from_array(logits)
+    for src in (dx.ptr, off.ptr + 4):
+        out, ids, w = gpu.DeviceBuffer(4 * hidden), gpu.DeviceBuffer(4 * top_k), gpu.DeviceBuffer(4 * top_k)
+        gpu.call("vbm_moe_layer_forward", C.byref(d), src, dl.ptr, 1, out.ptr, ids.ptr, w.ptr, work.ptr, need.value, None)
+        gpu.call("vbm_stream_synchronize", None)
+        assert np.array_equal(ids.download(np.int32, (1, top_k)), ref["ids"])
+        assert np.allclose(w.download(np.float32, (1, top_k)), ref["weights"], rtol=1e-6, atol=0)
+        got = out.download(np.float32, (1, hidden))
+        assert H.bits_equal(got, ref["out"]), H.diff_report(got, ref["out"])
+    layer.destroy()
