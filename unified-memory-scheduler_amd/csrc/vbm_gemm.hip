@@ -145,58 +145,6 @@ __device__ __forceinline__ half8_t i8_to_f16(long v) {
     for (int i = 0; i < 8; ++i) r[i] = static_cast<_Float16>(static_cast<signed char>(v >> (8 * i)));
     return r;
 }
-// Pipeline stages, filled by global-to-LDS DMA: a ring of S chunks of CB blocks, each stage
-// holding the job tile's activation codes and block scales of its chunk and, for MXFP4, both tiles'
-// weight dwords of those blocks ([slice][row] dwords, rows of odd slice pairs rotated by 16
-// against bank conflicts) and their exponent dword per row. Q8_0 (GROUPED): a tile's weights of
-// one 4-block bank group are 4 KB contiguous in the bank, so both tiles' group weights are staged
-// once per group by 16-byte DMAs into a two-slot group ring beside the chunk ring ([tile][slice]
-// [row] 16-byte units, the bank's own order), with the group's fp16 scales ([tile][row] 8 bytes)
-// and the job tile's activation block scales of the group ([job][4 blocks], 16 bytes each):
-// a third of the chunk's DMA instructions, whose issue (not their bytes) bounded the kernel
-// (doubling the weight DMAs of the former per-chunk dword staging added 55 us to a 345 us
-// gate_up launch, doubling the activation DMAs 30 us). The same group staging for MXFP4 (8-block
-// groups over four chunks, 2 waves per SIMD) measured slower, 1215-1280 against 1110-1136 us for
-// the MXFP4 gate_up of 2048 tokens top-4, so MXFP4 keeps per-chunk staging. Chunk c issues the loads of chunk c + 1
-// (and of the next group at its last chunk); one wait and one barrier per chunk. Two stages: a
-// third one, for every operand or for the weights alone, measured no faster (Q8_0 layer of 2048
-// tokens). Q8_0 chunks of a whole group (4 blocks, one barrier per group) need 132 VGPRs, so 3
-// instead of 4 workgroups per CU, and measured slower: 0.625 against 0.555 ms per layer.
-template <int TYPE>
-struct GemmStage {
-    static constexpr int kJobTile = job_tile<TYPE>();
-    static constexpr int EB = TYPE == 39 ? 2 : 1;                       // bytes per activation code
-    static constexpr int GB = TYPE == 39 ? 8 : 4;                       // blocks per bank group
-    static constexpr int CB = 2;                                        // blocks per chunk
-    static constexpr int CPG = GB / CB;                                 // chunks per group
-    static constexpr int S = 2;                                         // ring depth
-    static constexpr int ROW = CB * 32 * EB;                            // bytes per job row and chunk
-    static constexpr int ACT = kJobTile * ROW;
-    static constexpr bool GROUPED = TYPE == 8;
-    static constexpr int DA = GROUPED ? 0 : kJobTile * CB * 4;
-    static constexpr int W = GROUPED ? 0 : 2 * 8 * 32 * 4;
-    static constexpr int M = GROUPED ? 0 : 2 * 32 * 4;
-    static constexpr int OFF_DA = ACT, OFF_W = OFF_DA + DA, OFF_M = OFF_W + W;
-    static constexpr int STAGE = OFF_M + M;
-    static constexpr int WG = GROUPED ? 2 * 8 * 32 * 16 : 0;   // group weight slot: [tile][slice][row] x 16 B
-    static constexpr int MG = GROUPED ? 2 * 32 * 8 : 0;        // group scale slot: [tile][row] x 4 fp16
-    static constexpr int DG = GROUPED ? kJobTile * GB * 4 : 0;   // group block-scale slot: [job][4 blocks] fp32
-    static constexpr int OFF_WG = S * STAGE, OFF_MG = OFF_WG + 2 * WG, OFF_DG = OFF_MG + 2 * MG;
-    static constexpr int BYTES = OFF_DG + 2 * DG;
-    // DMA instructions per wave and chunk: activation rows (1 KiB each, ACT_JOBS job rows), block
-    // scales, weights, meta. A wave skips the activation loads whose job rows are all past the
-    // tile's live jobs, so its count per chunk varies; the wait before each chunk's barrier drains
-    // every load of the wave, which the two-stage ring allows (the next chunk's loads are issued
-    // after it).
-    static constexpr int ACT_JOBS = 1024 / ROW;
-    static constexpr int ACT_DMA = ACT / 1024 / 4;
-    static constexpr int W_DMA = W / 256 / 4;
-    static constexpr int WG_DMA = WG / 1024 / 4;   // 16-byte group weight loads per wave
-    static_assert(S == 2, "the per-chunk wait is vmcnt(0)");
-    static_assert(!GROUPED || (CPG == 2 && WG_DMA == 2), "Q8_0 group staging: two chunks per group, two loads per wave");
-    static_assert(ACT % 4096 == 0 && (!GROUPED || kJobTile % 64 == 0), "whole activation and block-scale DMAs per wave");
-};
-
 // Global-to-LDS DMA (global_load_lds_*): lane l's bytes land at LDS address m0 + l * size. The
 // loads are issued through inline assembly so that the compiler's wait-count pass, which would
 // wait for every such load before any LDS read it cannot prove disjoint, leaves the multi-stage
@@ -239,632 +187,6 @@ __device__ __forceinline__ float glu_fast(int activation, float g0, float u0, fl
     return __fdividef(g0, 1.0f + __expf(-g0)) * u0;
 }
 
-// fp16 x fp32 product on one instruction: v_fma_mix_f32 with the half in the low (HI = 0) or high
-// half of `h2` and -0 as the addend, i.e. exactly float(h) * x rounded once, signed zeros included.
-template <int HI>
-__device__ __forceinline__ float mul_half(unsigned h2, float x, float neg_zero) {
-    float r;
-    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(x), "s"(neg_zero));
-    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(x), "s"(neg_zero));
-    return r;
-}
-
-template <int TYPE, int EPI, bool FLAGGED>
-__global__ __launch_bounds__(kGemmThreads, (TYPE == 8 && !FLAGGED) ? 3 : 1) void grouped_gemm_kernel(GemmArgs A) {
-    using G = GemmStage<TYPE>;
-    constexpr int CB = G::CB;
-    constexpr int kJobTile = G::kJobTile;
-    constexpr int kLdsBytes = G::BYTES > kJobTile * 68 * 4 ? G::BYTES : kJobTile * 68 * 4;   // stages / epilogue tile
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
-    float (*tile_vals)[68] = reinterpret_cast<float (*)[68]>(lds);    // epilogue tile [job][pair row], after the K loop
-
-    // XCD-aware order: workgroup i runs on XCD i % 8, so hand each XCD a contiguous range of
-    // (tile, pair) items; the pairs of one job tile then share its activation rows in one L2 and
-    // consecutive tiles of an expert share its weights.
-    const int n_items = *cst<int32_t>(A.n_tiles) * A.row_pairs;
-    const int per_xcd = (n_items + 7) >> 3;
-    const int slot8 = static_cast<int>(blockIdx.x >> 3);
-    const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
-    if (slot8 >= per_xcd || item >= n_items) return;
-    const int ti = item / A.row_pairs;
-    const int pair = item - ti * A.row_pairs;
-    const int expert = cst<int32_t>(A.tile_expert)[ti];
-    const int j0 = cst<int32_t>(A.tile_start)[ti];
-    const int count = cst<int32_t>(A.counts)[expert];
-    const int joff = cst<int32_t>(A.offsets)[expert];
-    const int slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[expert] : expert;
-    const GemmShape S = A.shape;
-    if (slot < 0 || slot >= S.n_slots) {
-        // Expert not resident in this bank (a tile filter removes the experts a pass skips on
-        // purpose, so this is a bad map): this workgroup's outputs become NaN, as in the decode
-        // kernels, rather than leaving stale workspace data. Epilogue 1 poisons the block scale
-        // of the GLU block of this tile pair.
-        const float nan = __builtin_nanf("");
-        const int live_jobs = count - j0 < kJobTile ? count - j0 : kJobTile;
-        if (EPI == 0) {
-            for (int i = threadIdx.x; i < live_jobs * 64; i += kGemmThreads) {
-                const int64_t brow = static_cast<int64_t>(pair) * 64 + (i & 63);
-                if (brow < S.rows)
-                    A.dst[static_cast<size_t>(A.jobs[joff + j0 + (i >> 6)]) * S.rows + ggml_row(brow, S.rows, S.interleave)] = nan;
-            }
-        } else {
-            for (int j = threadIdx.x; j < live_jobs; j += kGemmThreads)
-                reinterpret_cast<float *>(A.rows_out + static_cast<int64_t>(A.jobs[joff + j0 + j]) * A.out_lay.stride() +
-                                          A.out_lay.da_offset())[pair] = nan;
-        }
-        return;
-    }
-
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int lr = lane & 15, q = lane >> 4;
-    const int tile = pair * 2 + (wave & 1);
-    const bool tile_live = tile * 32 < S.rows;
-    const int nb = S.nb;
-    const int groups = nb / G::GB, tail = nb % G::GB;
-    constexpr int kCodeRow = TYPE == 39 ? 16 : 32;     // code bytes per row and block
-    constexpr int kMetaRow = TYPE == 39 ? 1 : 2;       // exponent / scale bytes per row and block
-    const uint8_t * slot_base = A.bank + static_cast<size_t>(slot) * S.slot_bytes;
-    const uint8_t * codes = slot_base + static_cast<size_t>(tile_live ? tile : 0) * 32 * nb * kCodeRow;
-    const uint8_t * meta = slot_base + S.codes_bytes + static_cast<size_t>(tile_live ? tile : 0) * 32 * nb * kMetaRow;
-    auto row_of = [&](int jl) -> const uint8_t * {   // activation row of local job jl (must be live)
-        const int jb = A.jobs[joff + j0 + jl];
-        const int64_t row_index = A.b_ne1 == 1 ? jb / A.n_ids : jb;
-        return A.rows_in + row_index * A.lay.stride();
-    };
-
-    // The two wave halves (waves 0-1, 2-3) split the tile's live jobs at a multiple of 16: jobs
-    // [0, split) and [split, live), so a tile of n jobs costs each half about n / 2 of them (a
-    // 64-job tile gives each half 32 instead of all 64 to the first). This lane's fragment columns
-    // are jobs wj + 16jh + lr of its half; the -128 flags of the wave.
-    // Rows converted from caller-quantized Q8_0 data (FLAGGED) may hold -128 codes.
-    constexpr int JF = kJobTile / 32;
-    const int wq = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 7));   // the wave's half
-    const int live_jobs = count - j0 < kJobTile ? count - j0 : kJobTile;
-    const int split = 16 * ((live_jobs + 31) / 32);
-    const int wj = wq * split;                         // the wave's first job in the tile
-    const int half_end = wq ? live_jobs : (split < live_jobs ? split : live_jobs);
-    bool jlive[JF];
-    int flagged = 0;
-#pragma unroll
-    for (int jh = 0; jh < JF; ++jh) {
-        const int jl = wj + 16 * jh + lr;
-        jlive[jh] = jl < half_end;
-        if (FLAGGED && jlive[jh]) flagged |= *reinterpret_cast<const int *>(row_of(jl) + A.lay.flag_offset());
-    }
-    // Fragment columns of 16 jobs none of which is live (a half's live jobs are a prefix of it) cost
-    // the wave no matrix or scale work. The K loop is instantiated per count of live columns (nf,
-    // wave-uniform), so its body carries no per-column branch and the compiler can interleave the
-    // columns' MFMAs and VALU work.
-    static_assert(JF == 4 || JF == 6, "the K loop is instantiated for 0..6 live fragment columns");
-    const int live_in_half = half_end - wj;
-    const int nf = live_in_half <= 0 ? 0 : (live_in_half + 15) / 16;
-    // Workgroup-uniform: every wave then runs the same K-loop instantiation, so each of its
-    // barriers is reached from one control path (every thread gets here: the exits above are
-    // uniform per workgroup).
-    bool slow = false;
-    if constexpr (FLAGGED) slow = __syncthreads_or(flagged != 0) != 0;
-
-    // Stage loaders (global-to-LDS DMA). Lanes that have nothing to load are masked, and clamped
-    // sources keep every address inside the operands.
-    //   - activations: wave w's x4 loads j cover 16 (Q8_0) or 8 (MXFP4) job rows of the chunk;
-    //     the 16-byte parts of row r sit at part p ^ s(r) (s(r) = (r >> 1) & 3, resp. r & 7) so
-    //     the fragment reads of 16 consecutive rows spread over the banks; within a load that
-    //     holds a live job, a row past the tile's jobs reads the first job's row, and a load
-    //     whose rows are all past them is skipped (wave-uniform): those LDS rows keep stale
-    //     bytes, which reach only the matrix columns of jobs that are never stored;
-    //   - block scales: lane l of wave w loads job 32w + l / 2, block l % 2;
-    //   - weights: dword loads; Q8_0 load I = 4w + i covers tile I >> 3, slice pair (I >> 1) & 3,
-    //     rows 16 (I & 1) .. +15 (lane: row l >> 2, unit dword l & 3); MXFP4 load I = 2w + i covers
-    //     tile I >> 2, slices 2 (I & 3) and 2 (I & 3) + 1 (lane: slice l >> 5, position l & 31);
-    //     a tile past the bank's rows reads the pair's first tile (its rows are never stored);
-    //   - meta: lanes 0..15 of wave w load the dword of rows 16 (w & 1) .. +15 of tile w >> 1.
-    const int wu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int live_rows = __builtin_amdgcn_readfirstlane(count - j0);   // the tile's live jobs
-    // LDS address of the stage buffers: a generic pointer to LDS is the aperture base plus the
-    // LDS address in its low 32 bits.
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-    const uint8_t * act_src[G::ACT_DMA];
-#pragma unroll
-    for (int j = 0; j < G::ACT_DMA; ++j) {
-        const int jr = TYPE == 39 ? 8 * (wave * G::ACT_DMA + j) + (lane >> 3) : 16 * (wave * G::ACT_DMA + j) + (lane >> 2);
-        const int part = TYPE == 39 ? (lane & 7) ^ (jr & 7) : (lane & 3) ^ ((jr >> 1) & 3);
-        act_src[j] = row_of(j0 + jr < count ? jr : 0) + 16 * part;
-    }
-    // block scales: per chunk, lane l of wave w loads job 32w + l / 2, block l % 2; grouped (Q8_0),
-    // per group, lane l of waves w < kJobTile / 64 loads the 16 bytes of job 64w + l
-    static_assert(G::GROUPED || G::DA == kGemmThreads * 4, "one block-scale dword per thread and chunk");
-    const int jd = G::GROUPED ? 64 * (wave < kJobTile / 64 ? wave : 0) + lane : 32 * wave + (lane >> 1);
-    const uint8_t * da_src = row_of(j0 + jd < count ? jd : 0) + A.lay.da_offset() + (G::GROUPED ? 0 : 4 * (lane & 1));
-    // weight dword of this lane within its load's group-relative source
-    uint32_t woff;
-    if constexpr (TYPE == 39) {
-        const int k = lane >> 5, pos = lane & 31;            // slice within the pair of slices
-        woff = static_cast<uint32_t>((k * 32 + pos) * 16);   // the rotation depends on the pair: added per load
-    } else {
-        woff = static_cast<uint32_t>(((lane & 1) * 32 + (lane >> 2)) * 16 + 4 * ((lane >> 1) & 1));
-    }
-    const uint32_t moff = static_cast<uint32_t>(lane) * 8;
-    const size_t tile_bytes = static_cast<size_t>(32) * nb * kCodeRow, meta_tile_bytes = static_cast<size_t>(32) * nb * kMetaRow;
-    auto tsel = [&](int t) -> size_t { return (pair * 2 + t) * 32 < S.rows ? pair * 2 + t : pair * 2; };
-    // new_group: also stage chunk c's bank group (Q8_0), into group slot grp & 1; the slot of the
-    // group before it is still being read, the one before that is free since the barrier that
-    // ended its last chunk.
-    auto dma_stage = [&](int c, int st, bool new_group) {
-        const int grp = c / G::CPG, sub = c % G::CPG;
-        const uint32_t sb = lds0 + st * G::STAGE;
-#pragma unroll
-        for (int j = 0; j < G::ACT_DMA; ++j)
-            if (G::ACT_JOBS * (wu * G::ACT_DMA + j) < live_rows)
-                lds_dma_x4(act_src[j] + static_cast<int64_t>(c) * G::ROW, sb + (wu * G::ACT_DMA + j) * 1024);
-        if constexpr (!G::GROUPED) lds_dma_x1(da_src + static_cast<int64_t>(c) * CB * 4, sb + G::OFF_DA + wu * 256);
-        if constexpr (G::GROUPED) {
-            if (new_group) {
-                // load I = 2w + i: tile I >> 2, the 1 KiB quarter I & 3 of its group (lane l: the
-                // 16-byte unit 64 (I & 3) + l, i.e. slice 2 (I & 3) + l / 32, row l % 32)
-                const uint32_t wslot = lds0 + G::OFF_WG + (grp & 1) * G::WG;
-#pragma unroll
-                for (int i = 0; i < G::WG_DMA; ++i) {
-                    const int I = wu * G::WG_DMA + i, t = I >> 2, part = I & 3;
-                    const uint8_t * base = slot_base + tsel(t) * tile_bytes + static_cast<size_t>(grp) * 4096 + part * 1024;
-                    lds_dma_x4_s(base, static_cast<uint32_t>(lane) * 16, wslot + t * 4096 + part * 1024);
-                }
-                // the group's scales: lanes 0..31 of wave 0, 16 bytes (two rows) each, tile l / 16
-                if (wu == 0 && lane < 32)
-                    lds_dma_x4(slot_base + S.codes_bytes + tsel(lane >> 4) * meta_tile_bytes + static_cast<size_t>(grp) * 256 +
-                                   (lane & 15) * 16,
-                               lds0 + G::OFF_MG + (grp & 1) * G::MG);
-                if (wu < kJobTile / 64)
-                    lds_dma_x4(da_src + 16 * grp,
-                               __builtin_amdgcn_readfirstlane(lds0 + G::OFF_DG + (grp & 1) * G::DG + wu * 1024));
-            }
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < G::W_DMA; ++i) {
-            const int I = wu * G::W_DMA + i;
-            if constexpr (TYPE == 39) {
-                // slices 2 (I & 3) + (l >> 5): odd slice pairs hold row r at position r ^ 16
-                const int t = I >> 2, kp = I & 3;
-                const uint8_t * base = slot_base + tsel(t) * tile_bytes + static_cast<size_t>(grp) * 4096 + kp * 2 * 512 + 4 * sub;
-                lds_dma_x1_s(base, (kp & 1) ? (woff ^ (16 * 16)) : woff, sb + G::OFF_W + (t * 8 + kp * 2) * 128);
-            } else {
-                const int t = I >> 3, qq = (I >> 1) & 3, rh = I & 1;
-                const uint8_t * base =
-                    slot_base + tsel(t) * tile_bytes + static_cast<size_t>(grp) * 4096 + (2 * qq * 32 + rh * 16) * 16 + 8 * sub;
-                lds_dma_x1_s(base, woff, sb + G::OFF_W + t * 2048 + (qq * 32 + rh * 16) * 16);
-            }
-        }
-        const uint8_t * mbase = slot_base + S.codes_bytes + tsel(wu >> 1) * meta_tile_bytes + static_cast<size_t>(grp) * 256 +
-                                16 * (wu & 1) * 8 + (TYPE == 39 ? 4 * (sub >> 1) : 4 * sub);
-        if (lane < 16) lds_dma_x1_s(mbase, moff, sb + G::OFF_M + wu * 64);
-    };
-
-    f32x4 acc[2][JF];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int jh = 0; jh < JF; ++jh) acc[i][jh] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // One block: weight operands a_op[i] (row halves i), activation operand and scale of job half
-    // jh from bsrc(jh) / dsrc(jh); factor(i, j, da) is the block's fp32 scale for output row
-    // 16i + 4q + j: ldexp(da, e) for MXFP4 exponent e, fp16(d_w) * da for Q8_0. SLOW adds the
-    // exact -128 correction, accumulated into the same MFMA result (its operands scaled by 256
-    // are exact in fp16).
-    const float neg_zero = -0.0f;
-    auto block_step = [&](auto slow_c, auto nf_c, const auto & a_op, auto && factor, auto && bsrc, auto && dsrc) {
-        constexpr bool SLOW = decltype(slow_c)::value;
-        constexpr int NF = decltype(nf_c)::value;
-#pragma unroll
-        for (int jh = 0; jh < NF; ++jh) {
-            const float da = dsrc(jh);
-            const auto bv = bsrc(jh);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                f32x4 d;
-                if constexpr (TYPE == 39) {
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op[i], bv, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    if constexpr (SLOW) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(neg_part(a_op[i]), is_neg128_x256(bv), d, 0, 0, 0);
-                } else if constexpr (!SLOW) {
-                    const i32x4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_op[i], bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) d[j] = static_cast<float>(di[j]);
-                } else {
-                    const half8_t a16 = i8_to_f16(a_op[i]), b16 = i8_to_f16(bv);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a16, b16, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(neg_part(a16), is_neg128_x256(b16), d, 0, 0, 0);
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][jh][j] = __builtin_fmaf(factor(i, j, da), d[j], acc[i][jh][j]);
-            }
-        }
-    };
-
-    // The K loop, instantiated with and without the -128 correction (workgroup-uniform choice) and
-    // per count of live fragment columns.
-    const int n_chunks = groups * G::CPG;
-    auto k_loop = [&](auto slow_c, auto nf_c) {
-        constexpr int NF = decltype(nf_c)::value;
-        // weight dwords of A rows lr + 16i, slices 2q / 2q + 1 (MXFP4: row r of an odd slice pair
-        // at position r ^ 16), or their 16-byte unit (Q8_0)
-        // (Q8_0: unit (2q, row) of the group slot; slice 2q + 1's unit is 512 bytes on)
-        const uint8_t * w_lds[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            w_lds[i] = TYPE == 39 ? lds + G::OFF_W + ((wave & 1) * 256 + 2 * q * 32 + 16 * (i ^ (q & 1)) + lr) * 4
-                                  : lds + G::OFF_WG + (wave & 1) * 4096 + (2 * q * 32 + 16 * i + lr) * 16;
-        // exponent dword (MXFP4, per chunk stage) or the group's 8 scale bytes (Q8_0, group slot)
-        // of output rows 4q + j (+16i) and of A rows lr (+16i)
-        const uint8_t * m_lds = TYPE == 39 ? lds + G::OFF_M + ((wave & 1) * 32 + 4 * q) * 4
-                                           : lds + G::OFF_MG + ((wave & 1) * 32 + 4 * q) * 8;
-        const uint8_t * ma_lds = TYPE == 39 ? lds + G::OFF_M + ((wave & 1) * 32 + lr) * 4
-                                            : lds + G::OFF_MG + ((wave & 1) * 32 + lr) * 8;
-        const float * d_lds = G::GROUPED ? reinterpret_cast<const float *>(lds + G::OFF_DG) + (wj + lr) * G::GB
-                                         : reinterpret_cast<const float *>(lds + G::OFF_DA) + (wj + lr) * CB;
-        // fragment columns' activation codes: row rr = wj + 16jh + lr, block bb, codes 8q..8q+7
-        uint32_t aoff[JF][2];
-#pragma unroll
-        for (int jh = 0; jh < JF; ++jh)
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb) {
-                const int rr = wj + 16 * jh + lr;
-                aoff[jh][bb] = TYPE == 39 ? rr * 128 + (((4 * bb + q) ^ (rr & 7)) << 4)
-                                          : rr * 64 + (((2 * bb + (q >> 1)) ^ ((rr >> 1) & 3)) << 4) + 8 * (q & 1);
-            }
-#pragma clang loop unroll(disable)
-        for (int c = 0; c < n_chunks; ++c) {
-            const int sub = c % G::CPG, gs = (c / G::CPG) & 1;   // gs: this chunk's group slot
-            // this chunk's loads: the stage of chunk c + 1, clamped to the last chunk (the stage
-            // it fills is free either way), and chunk c + 1's bank group when it starts one
-            dma_stage(c + 1 < n_chunks ? c + 1 : n_chunks - 1, (c + 1) % G::S, c + 1 < n_chunks && (c + 1) % G::CPG == 0);
-            const int ab = c % G::S, wb = ab;
-            const uint8_t * st = lds + ab * G::STAGE;     // this chunk's stage
-            // This chunk's blocks 2sub, 2sub+1 in the group: weight dwords of slices 2q, 2q+1
-            // (MXFP4: one dword holds both blocks; Q8_0: one dword each).
-            unsigned w0[2][2], w1[2][2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if constexpr (TYPE == 39) {
-                    const uint8_t * w = w_lds[i] + wb * G::STAGE;
-                    w0[i][0] = w0[i][1] = *reinterpret_cast<const unsigned *>(w);
-                    w1[i][0] = w1[i][1] = *reinterpret_cast<const unsigned *>(w + 32 * 4);
-                } else {
-                    const uint8_t * w = w_lds[i] + gs * G::WG + 8 * sub;
-                    const u32x2g a = *reinterpret_cast<const u32x2g *>(w), b = *reinterpret_cast<const u32x2g *>(w + 512);
-                    w0[i][0] = a[0], w0[i][1] = a[1], w1[i][0] = b[0], w1[i][1] = b[1];
-                }
-            }
-            // MXFP4 fast path: when every exponent e of the wave's A rows (16i + lr) lies in
-            // [-14, 12], 2^(e+1) times the e2m1 values is an exact normal f16, so the exponent
-            // rides in the A operand and the block result needs one FMA with d_act:
-            // da * (2^e * dot) rounds the same product as ldexp(da, e) * dot.
-            bool folded = false;
-            float fsc[2][2];
-            if constexpr (TYPE == 39 && !decltype(slow_c)::value) {
-                bool ok = true;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const unsigned ea = *reinterpret_cast<const uint16_t *>(ma_lds + wb * G::STAGE + i * 16 * 4 + (sub & 1) * 2);
-#pragma unroll
-                    for (int bb = 0; bb < 2; ++bb) {
-                        const int e = static_cast<signed char>(ea >> (8 * bb));
-                        ok = ok && e >= -14 && e <= 12;
-                        fsc[i][bb] = __builtin_bit_cast(float, static_cast<unsigned>(e + 128) << 23);
-                    }
-                }
-                folded = __all(ok);
-            }
-            if (folded) {
-#pragma unroll
-                for (int bb = 0; bb < CB; ++bb) {
-                    half8_t a_op[2];
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) a_op[i] = mx_a_operand(w0[i][bb], w1[i][bb], bb, fsc[i][bb]);
-#pragma unroll
-                    for (int jh = 0; jh < NF; ++jh) {
-                        const float da = d_lds[ab * (G::STAGE / 4) + 16 * jh * CB + bb];
-                        const half8_t bv = *reinterpret_cast<const half8_t *>(st + aoff[jh][bb]);
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) {
-                            const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_op[i], bv, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) acc[i][jh][j] = __builtin_fmaf(da, d[j], acc[i][jh][j]);
-                        }
-                    }
-                }
-            } else if constexpr (TYPE == 8 && !decltype(slow_c)::value) {
-                // Q8_0: the scale products fp16(d_w) * d_act of a 16 x 16 output fragment come
-                // from one f16 MFMA per block: A holds d_w of the fragment's 16 rows at k = bb
-                // (lanes 0..15, zero elsewhere), B the 16 jobs' d_act at k = bb. Each output is
-                // the exact fp32 product of two fp16 values (11-bit significands) plus zeros:
-                // the value the per-output VALU product gives, off the vector ALU.
-                const unsigned sel[2] = {lane < 16 ? 0x0000FFFFu : 0u, lane < 16 ? 0xFFFF0000u : 0u};
-                unsigned dw_row[2], da_pk[JF];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) dw_row[i] = *reinterpret_cast<const unsigned *>(ma_lds + gs * G::MG + i * 16 * 8 + 4 * sub);
-#pragma unroll
-                for (int jh = 0; jh < NF; ++jh) {
-                    // d_act holds fp16 values, so the packing conversion is exact
-                    const float * dp = d_lds + gs * (G::DG / 4) + 16 * jh * G::GB + CB * sub;
-                    da_pk[jh] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(dp[0], dp[1]));
-                }
-#pragma unroll
-                for (int bb = 0; bb < CB; ++bb) {
-                    long a_op[2];
-                    half4_g as[2];
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        a_op[i] = static_cast<long>(static_cast<uint64_t>(w0[i][bb]) | (static_cast<uint64_t>(w1[i][bb]) << 32));
-                        as[i] = __builtin_bit_cast(half4_g, u32x2g{dw_row[i] & sel[bb], 0u});
-                    }
-#pragma unroll
-                    for (int jh = 0; jh < NF; ++jh) {
-                        const long bv = *reinterpret_cast<const long *>(st + aoff[jh][bb]);
-                        const half4_g bs = __builtin_bit_cast(half4_g, u32x2g{da_pk[jh] & sel[bb], 0u});
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) {
-                            const i32x4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_op[i], bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
-                            const f32x4 sc = __builtin_amdgcn_mfma_f32_16x16x16f16(as[i], bs, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                acc[i][jh][j] = __builtin_fmaf(sc[j], static_cast<float>(di[j]), acc[i][jh][j]);
-                        }
-                    }
-                }
-            } else {
-                // exponent / scale bytes of output rows 16i + 4q + j (MXFP4 one byte, Q8_0 two per block)
-                // (Q8_0: both blocks' fp16 scales of a row in one dword)
-                unsigned mw[2][4];
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if constexpr (TYPE == 39)
-                            mw[i][j] = *reinterpret_cast<const uint16_t *>(m_lds + wb * G::STAGE + (16 * i + j) * 4 + (sub & 1) * 2);
-                        else
-                            mw[i][j] = *reinterpret_cast<const unsigned *>(m_lds + gs * G::MG + (16 * i + j) * 8 + 4 * sub);
-                    }
-                auto do_block = [&](int bb) {
-                    auto bsrc = [&](int jh) {
-                        const uint8_t * p = st + aoff[jh][bb];
-                        if constexpr (TYPE == 39) return *reinterpret_cast<const half8_t *>(p);
-                        else return *reinterpret_cast<const long *>(p);
-                    };
-                    auto dsrc = [&](int jh) {
-                        if constexpr (G::GROUPED) return d_lds[gs * (G::DG / 4) + 16 * jh * G::GB + CB * sub + bb];
-                        else return d_lds[ab * (G::STAGE / 4) + 16 * jh * CB + bb];
-                    };
-                    if constexpr (TYPE == 39) {
-                        auto factor = [&](int i, int j, float da) {
-                            return __builtin_amdgcn_ldexpf(da, static_cast<signed char>(mw[i][j] >> (8 * bb)));
-                        };
-                        half8_t a_op[2];
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) a_op[i] = mx_a_operand(w0[i][bb], w1[i][bb], bb);
-                        block_step(slow_c, nf_c, a_op, factor, bsrc, dsrc);
-                    } else {
-                        auto factor = [&](int i, int j, float da) {
-                            return bb ? mul_half<1>(mw[i][j], da, neg_zero) : mul_half<0>(mw[i][j], da, neg_zero);
-                        };
-                        long a_op[2];
-#pragma unroll
-                        for (int i = 0; i < 2; ++i)
-                            a_op[i] = static_cast<long>(static_cast<uint64_t>(w0[i][bb]) | (static_cast<uint64_t>(w1[i][bb]) << 32));
-                        block_step(slow_c, nf_c, a_op, factor, bsrc, dsrc);
-                    }
-                };
-                if constexpr (decltype(slow_c)::value) {
-#pragma clang loop unroll(disable)
-                    for (int bb = 0; bb < CB; ++bb) do_block(bb);
-                } else {
-#pragma unroll
-                    for (int bb = 0; bb < CB; ++bb) do_block(bb);
-                }
-            }
-            // the stage of chunk c + 1, issued at the top of this chunk
-            lds_dma_wait<0>();
-            __syncthreads();
-        }
-
-        // Tail blocks (nb even: MXFP4 tail in {0,2,4,6}, Q8_0 tail in {0,2}), per-row packed, read
-        // straight from global memory.
-        for (int bt = 0; bt < tail; ++bt) {
-            const int b = groups * G::GB + bt;
-            unsigned m[2][4];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int orow = 16 * i + 4 * q + j;
-                    m[i][j] = 0;
-                    if (tile_live) {
-                        if constexpr (TYPE == 39) m[i][j] = meta[groups * 256 + orow * tail + bt];
-                        else m[i][j] = *reinterpret_cast<const uint16_t *>(meta + groups * 256 + (orow * tail + bt) * 2);
-                    }
-                }
-            auto factor = [&](int i, int j, float da) {
-                if constexpr (TYPE == 39) return __builtin_amdgcn_ldexpf(da, static_cast<signed char>(m[i][j]));
-                else return half_bits_to_float(static_cast<uint16_t>(m[i][j])) * da;
-            };
-            const uint8_t * brow[JF];
-#pragma unroll
-            for (int jh = 0; jh < JF; ++jh) brow[jh] = jlive[jh] ? row_of(wj + 16 * jh + lr) : nullptr;
-            auto bsrc = [&](int jh) {
-                if constexpr (TYPE == 39) {
-                    half8_t v = half8_t{};
-                    if (brow[jh]) v = *reinterpret_cast<const half8_t *>(brow[jh] + (static_cast<int64_t>(b) * 32 + 8 * q) * 2);
-                    return v;
-                } else {
-                    long v = 0;
-                    if (brow[jh]) v = *reinterpret_cast<const long *>(brow[jh] + static_cast<int64_t>(b) * 32 + 8 * q);
-                    return v;
-                }
-            };
-            auto dsrc = [&](int jh) { return brow[jh] ? reinterpret_cast<const float *>(brow[jh] + A.lay.da_offset())[b] : 0.0f; };
-            if constexpr (TYPE == 39) {
-                half8_t a[2];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int r = 16 * i + lr;
-                    unsigned w0 = 0, w1 = 0;
-                    if (tile_live) {
-                        w0 = *reinterpret_cast<const uint16_t *>(codes + groups * 4096 + ((2 * q) * 32 + r) * (tail * 2) + bt * 2);
-                        w1 = *reinterpret_cast<const uint16_t *>(codes + groups * 4096 + ((2 * q + 1) * 32 + r) * (tail * 2) + bt * 2);
-                    }
-                    const half2_g p0 = fp4x2(w0, 0), p1 = fp4x2(w0, 1), p2 = fp4x2(w1, 0), p3 = fp4x2(w1, 1);
-                    a[i] = half8_t{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
-                }
-                block_step(slow_c, nf_c, a, factor, bsrc, dsrc);
-            } else {
-                long a[2];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int r = 16 * i + lr;
-                    uint64_t w0 = 0, w1 = 0;
-                    if (tile_live) {
-                        w0 = *reinterpret_cast<const unsigned *>(codes + groups * 4096 + ((2 * q) * 32 + r) * (tail * 4) + bt * 4);
-                        w1 = *reinterpret_cast<const unsigned *>(codes + groups * 4096 + ((2 * q + 1) * 32 + r) * (tail * 4) + bt * 4);
-                    }
-                    a[i] = static_cast<long>(w0 | (w1 << 32));
-                }
-                block_step(slow_c, nf_c, a, factor, bsrc, dsrc);
-            }
-        }
-    };
-    // Prologue: stages 0 .. S - 2 (clamped).
-    if (groups > 0) {
-        dma_stage(0, 0, true);
-        lds_dma_wait<0>();
-    }
-    __syncthreads();
-    // Waves of one workgroup may take different instantiations (their job halves hold different
-    // numbers of live columns); every instantiation issues the same stage loads and reaches one
-    // barrier per chunk.
-    auto k_loop_nf = [&](auto slow_c) {
-        switch (nf) {
-            case 6: if constexpr (JF >= 6) k_loop(slow_c, std::integral_constant<int, 6>{}); break;
-            case 5: if constexpr (JF >= 5) k_loop(slow_c, std::integral_constant<int, 5>{}); break;
-            case 4: k_loop(slow_c, std::integral_constant<int, 4>{}); break;
-            case 3: k_loop(slow_c, std::integral_constant<int, 3>{}); break;
-            case 2: k_loop(slow_c, std::integral_constant<int, 2>{}); break;
-            case 1: k_loop(slow_c, std::integral_constant<int, 1>{}); break;
-            default: k_loop(slow_c, std::integral_constant<int, 0>{}); break;
-        }
-    };
-    if constexpr (FLAGGED) {
-        if (slow) k_loop_nf(std::true_type{});
-        else k_loop_nf(std::false_type{});
-    } else {
-        k_loop_nf(std::false_type{});
-    }
-    // The clamped loads of the last chunks may still be landing in the stages the epilogue reuses.
-    lds_dma_wait<0>();
-    __syncthreads();
-
-    // Epilogue: biases (ggml row order), then either fp32 rows (times the job's routing weight when
-    // row_scale is given: ggml's ADD_ID, then MUL, hybrid-experts.patch:1636-1646) or GLU + Q8_0
-    // requantization. The fp32 rows go through the LDS tile too when the output allows 16-byte
-    // stores, so that each job's 64 rows leave as four full 64-byte segments instead of 4-byte
-    // scatter.
-    const bool via_lds = EPI == 1 || A.dst_vec4;
-    // the fragment columns' jobs and routing weights, loaded only now (held through the K loop they
-    // cost registers it needs)
-    int job[JF];
-    float rscale[JF];
-#pragma unroll
-    for (int jh = 0; jh < JF; ++jh) {
-        job[jh] = jlive[jh] ? A.jobs[joff + j0 + wj + 16 * jh + lr] : 0;
-        rscale[jh] = EPI == 0 && A.row_scale && jlive[jh] ? A.row_scale[job[jh]] : 1.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int orow = 16 * i + 4 * q + j;
-            const int grow = static_cast<int>(ggml_row(static_cast<int64_t>(tile) * 32 + orow, S.rows, S.interleave));
-            const float bv = (A.bias && tile_live) ? A.bias[static_cast<size_t>(expert) * S.rows + grow] : 0.0f;
-#pragma unroll
-            for (int jh = 0; jh < JF; ++jh) {
-                float v = acc[i][jh][j];
-                if (A.bias) v = v + bv;
-                if (EPI == 0 && A.row_scale) v = v * rscale[jh];
-                if (!via_lds) {
-                    if (jlive[jh] && tile_live) A.dst[static_cast<size_t>(job[jh]) * S.rows + grow] = v;
-                } else if (jlive[jh]) {   // columns past the half's jobs belong to the other half
-                    tile_vals[wj + 16 * jh + lr][32 * (wave & 1) + orow] = v;
-                }
-            }
-        }
-    }
-    if (!via_lds) return;
-    __syncthreads();
-    for (int jl = threadIdx.x >> 2; jl < kJobTile; jl += kGemmThreads / 4) {   // four threads per job
-        const int jj = j0 + jl;
-        if (EPI == 0) {
-            // 16 pair rows per thread; aligned runs of 4 device rows are 4 consecutive ggml rows
-            // (also in interleaved gate|up banks)
-            const int seg = threadIdx.x & 3;
-            if (jj < count) {
-                float * out = A.dst + static_cast<size_t>(A.jobs[joff + jj]) * S.rows;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int col = seg * 16 + 4 * k;
-                    const int64_t brow = static_cast<int64_t>(pair) * 64 + col;
-                    if (brow < S.rows)
-                        *reinterpret_cast<float4 *>(out + ggml_row(brow, S.rows, S.interleave)) =
-                            *reinterpret_cast<const float4 *>(&tile_vals[jl][col]);
-                }
-            }
-        } else {
-            // one 32-element GLU block per job, eight elements per thread
-            const int part = threadIdx.x & 3;
-            const bool live = jj < count;
-            float x[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int e = part * 8 + t;                 // element of the block
-                const int tl = e >> 4;                      // bank tile of the pair
-                const float g = tile_vals[jl][32 * tl + (e & 15)];
-                const float u = tile_vals[jl][32 * tl + 16 + (e & 15)];
-                x[t] = glu_fast(A.activation, g, u, A.alpha, A.limit);
-            }
-            float amax = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf(x[t]));
-            amax = quad_max(amax);
-            if (live) {
-                const float d = amax / 127.0f;
-                const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
-                const int jb = A.jobs[joff + jj];
-                uint8_t * out = A.rows_out + static_cast<int64_t>(jb) * A.out_lay.stride();
-                const int64_t e0 = static_cast<int64_t>(pair) * 32 + part * 8;
-                if (A.out_lay.weight_type == 39) {
-                    half8_t c;
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        float v = rintf(x[t] * id);
-                        v = v > 127.0f ? 127.0f : (v < -128.0f ? -128.0f : v);
-                        c[t] = static_cast<_Float16>(v);
-                    }
-                    *reinterpret_cast<half8_t *>(out + e0 * 2) = c;
-                } else {
-                    uint64_t c = 0;
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        float v = rintf(x[t] * id);
-                        v = v > 127.0f ? 127.0f : (v < -128.0f ? -128.0f : v);
-                        c |= static_cast<uint64_t>(static_cast<uint8_t>(static_cast<signed char>(v))) << (8 * t);
-                    }
-                    *reinterpret_cast<uint64_t *>(out + e0) = c;
-                }
-                if (part == 0) {
-                    reinterpret_cast<float *>(out + A.out_lay.da_offset())[pair] = static_cast<float>(static_cast<_Float16>(d));
-                    if (pair == 0) *reinterpret_cast<int *>(out + A.out_lay.flag_offset()) = 0;   // never -128
-                }
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------------ MXFP4 grouped GEMM
 // A wave owns 64 bank rows (a tile pair, so a whole 32-element GLU block of an interleaved bank) and
 // up to 64 jobs: a 4 x 4 grid of 16 x 16 fragments. Its weights go from the bank straight into
@@ -901,59 +223,174 @@ __device__ __forceinline__ unsigned mx_unfoldable(unsigned w) {
     return (((lo + 0x0E0E0E0Eu) ^ sg) | ((lo + 0x13131313u) ^ sg)) & 0xE0E0E0E0u;
 }
 
-template <int EPI, bool FLAGGED>
-__global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs A) {
-    using L = MxStageLayout;
-    __shared__ __attribute__((aligned(256))) uint8_t lds[L::BYTES];
-    // XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of
-    // (tile, row unit) items; the units of one job tile share its activation rows in one L2.
+// A workgroup's work in the grouped GEMMs below: 256 rows (four tile pairs from pair0) of one expert x the
+// live jobs of one job tile.
+struct RowsItem {
+    int expert, j0, joff, live, slot, pair0;
+};
+
+// XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of (tile, row unit)
+// items; the units of one job tile share its activation rows in one L2. False: no item, or one whose
+// expert is not resident in this bank. The latter writes NaN outputs, as the decode kernels do (a tile
+// filter removes the experts a pass skips on purpose, so this is a bad map).
+template <int EPI>
+__device__ __forceinline__ bool rows_item(const GemmArgs & A, int job_tile, RowsItem & it) {
     const int n_items = *cst<int32_t>(A.n_tiles) * A.row_units;
     const int per_xcd = (n_items + 7) >> 3;
     const int slot8 = static_cast<int>(blockIdx.x >> 3);
     const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
-    if (slot8 >= per_xcd || item >= n_items) return;
+    if (slot8 >= per_xcd || item >= n_items) return false;
     const int ti = item / A.row_units;
-    const int unit = item - ti * A.row_units;
-    const int expert = cst<int32_t>(A.tile_expert)[ti];
-    const int j0 = cst<int32_t>(A.tile_start)[ti];
-    const int count = cst<int32_t>(A.counts)[expert];
-    const int joff = cst<int32_t>(A.offsets)[expert];
-    const int slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[expert] : expert;
-    const GemmShape S = A.shape;
-    const int live = count - j0 < L::kJobs ? count - j0 : L::kJobs;
-    const int pair0 = unit * 4, n_pairs = 4;
-    if (slot < 0 || slot >= S.n_slots) {
-        // Expert not resident in this bank: NaN outputs, as in the decode kernels (a tile filter
-        // removes the experts a pass skips on purpose, so this is a bad map).
-        const float nan = __builtin_nanf("");
-        if (EPI == 0) {
-            for (int i = threadIdx.x; i < live * n_pairs * 64; i += kGemmThreads) {
-                const int64_t brow = static_cast<int64_t>(pair0) * 64 + i % (n_pairs * 64);
-                if (brow < S.rows)
-                    A.dst[static_cast<size_t>(A.jobs[joff + j0 + i / (n_pairs * 64)]) * S.rows + ggml_row(brow, S.rows, S.interleave)] = nan;
+    it.pair0 = (item - ti * A.row_units) * 4;
+    it.expert = cst<int32_t>(A.tile_expert)[ti];
+    it.j0 = cst<int32_t>(A.tile_start)[ti];
+    const int count = cst<int32_t>(A.counts)[it.expert];
+    it.joff = cst<int32_t>(A.offsets)[it.expert];
+    it.slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[it.expert] : it.expert;
+    it.live = count - it.j0 < job_tile ? count - it.j0 : job_tile;
+    const GemmShape & S = A.shape;
+    if (it.slot >= 0 && it.slot < S.n_slots) return true;
+    const float nan = __builtin_nanf("");
+    if (EPI == 0) {
+        for (int i = threadIdx.x; i < it.live * 256; i += kGemmThreads) {
+            const int64_t brow = static_cast<int64_t>(it.pair0) * 64 + i % 256;
+            if (brow < S.rows)
+                A.dst[static_cast<size_t>(A.jobs[it.joff + it.j0 + i / 256]) * S.rows + ggml_row(brow, S.rows, S.interleave)] = nan;
+        }
+    } else {
+        for (int i = threadIdx.x; i < it.live * 4; i += kGemmThreads)
+            if ((it.pair0 + i % 4) * 64 < S.rows)
+                reinterpret_cast<float *>(A.rows_out + static_cast<int64_t>(A.jobs[it.joff + it.j0 + i / 4]) * A.out_lay.stride() +
+                                          A.out_lay.da_offset())[it.pair0 + i % 4] = nan;
+    }
+    return false;
+}
+
+// Byte address of 16-byte unit `off` of `base`.
+__device__ __forceinline__ const uint8_t * unit_ptr(const uint8_t * base, uint32_t off) { return base + static_cast<uint64_t>(off) * 16; }
+
+// Row offset of live local job jl, in 16-byte units.
+__device__ __forceinline__ uint32_t row_off16(const GemmArgs & A, const RowsItem & it, int jl) {
+    const uint32_t jb = static_cast<uint32_t>(A.jobs[it.joff + it.j0 + jl]);
+    const uint32_t row = A.b_ne1 == 1 ? jb / static_cast<uint32_t>(A.n_ids) : jb;
+    return row * static_cast<uint32_t>(A.lay.stride() / 16);
+}
+
+// Epilogue, from registers: lane (q, lr) holds rows 16i + 4q .. + 3 of tile pair `pair` for job 16jh + lr, jh < nf.
+// Biases (ggml row order), then fp32 rows (times the routing weight when given) as one 16-byte store per
+// fragment, or GLU + Q8_0 requantization: fragments 0 / 1 and 2 / 3 are the gate / up rows of the block's
+// elements 4q .. + 3 and 16 + 4q .. + 3.
+template <int TYPE, int EPI>
+__device__ __forceinline__ void rows_epilogue(const GemmArgs & A, const RowsItem & it, int pair, int nf, const f32x4 (&acc)[4][4]) {
+    const GemmShape & S = A.shape;
+    const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+    const bool two_tiles = pair * 64 + 32 < S.rows;          // the last pair may be one tile
+    // ggml rows of the lane's fragments: aligned runs of 4 device rows are 4 consecutive ggml rows, also in
+    // interleaved banks (tile 2 pair + i / 2; its rows 16.. are the up rows there)
+    uint32_t grow[4];
+    float bias[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        grow[i] = S.interleave ? static_cast<uint32_t>((i & 1) * (S.rows / 2) + (2 * pair + (i >> 1)) * 16 + 4 * q)
+                               : static_cast<uint32_t>(64 * pair + 16 * i + 4 * q);
+        const bool row_live = i < 2 || two_tiles;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias[i][j] = A.bias && row_live ? A.bias[static_cast<size_t>(it.expert) * S.rows + grow[i] + j] : 0.0f;
+    }
+    int jobs[4];
+    float scales[4];
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) jobs[jh] = A.jobs[it.joff + it.j0 + (16 * jh + lr < it.live ? 16 * jh + lr : 0)];
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) scales[jh] = EPI == 0 && A.row_scale ? A.row_scale[jobs[jh]] : 1.0f;
+#pragma unroll
+    for (int jh = 0; jh < 4; ++jh) {
+        if (jh >= nf) break;
+        const bool jlive = 16 * jh + lr < it.live;
+        const int job = jobs[jh];
+        if constexpr (EPI == 0) {
+            const float rs = scales[jh];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!jlive || (i >= 2 && !two_tiles)) continue;
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[j] = acc[i][jh][j];
+                    if (A.bias) v[j] = v[j] + bias[i][j];
+                    if (A.row_scale) v[j] = v[j] * rs;
+                }
+                float * out = A.dst + static_cast<size_t>(job) * S.rows + grow[i];
+                if (A.dst_vec4) {
+                    f32x4 vv = {v[0], v[1], v[2], v[3]};
+                    asm volatile("" : "+v"(vv));             // (merged with the scalar form it becomes dword stores)
+                    *reinterpret_cast<f32x4 *>(out) = vv;
+                } else {
+                    asm volatile("" : "+v"(out));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) out[j] = v[j];
+                }
             }
         } else {
-            for (int i = threadIdx.x; i < live * n_pairs; i += kGemmThreads)
-                if ((pair0 + i % n_pairs) * 64 < S.rows)
-                    reinterpret_cast<float *>(A.rows_out + static_cast<int64_t>(A.jobs[joff + j0 + i / n_pairs]) * A.out_lay.stride() +
-                                              A.out_lay.da_offset())[pair0 + i % n_pairs] = nan;
+            float x[2][4], amax = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float gv = acc[2 * t][jh][j], uv = acc[2 * t + 1][jh][j];
+                    if (A.bias) gv = gv + bias[2 * t][j], uv = uv + bias[2 * t + 1][j];
+                    x[t][j] = glu_fast(A.activation, gv, uv, A.alpha, A.limit);
+                    amax = fmaxf(amax, fabsf(x[t][j]));
+                }
+            amax = fmaxf(amax, __shfl_xor(amax, 16));        // the block's other lanes of this job
+            amax = fmaxf(amax, __shfl_xor(amax, 32));
+            const float d = amax / 127.0f;
+            const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+            if (!jlive) continue;
+            uint8_t * out = A.rows_out + static_cast<int64_t>(job) * A.out_lay.stride();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                half4_g c;
+                unsigned c8 = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v = rintf(x[t][j] * id);
+                    v = v > 127.0f ? 127.0f : (v < -128.0f ? -128.0f : v);
+                    if (TYPE == 39) c[j] = static_cast<_Float16>(v);
+                    else c8 |= static_cast<unsigned>(static_cast<uint8_t>(static_cast<signed char>(v))) << (8 * j);
+                }
+                const int64_t e0 = static_cast<int64_t>(pair) * 32 + 16 * t + 4 * q;
+                if (TYPE == 39) *reinterpret_cast<half4_g *>(out + e0 * 2) = c;
+                else *reinterpret_cast<unsigned *>(out + e0) = c8;
+            }
+            if (q == 0) {
+                reinterpret_cast<float *>(out + A.out_lay.da_offset())[pair] = static_cast<float>(static_cast<_Float16>(d));
+                if (pair == 0) *reinterpret_cast<int *>(out + A.out_lay.flag_offset()) = 0;   // never -128
+            }
         }
-        return;
     }
+}
 
+template <int EPI, bool FLAGGED>
+__global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs A) {
+    using L = MxStageLayout;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[L::BYTES];
+    RowsItem it;
+    if (!rows_item<EPI>(A, L::kJobs, it)) return;
+    const GemmShape S = A.shape;
+    const int live = it.live;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int lr = lane & 15, q = lane >> 4;
     const int nb = S.nb, groups = nb / 8, tail = nb % 8;
     const int n_groups = groups + (tail ? 1 : 0);
-    const int pair = pair0 + wave;
+    const int pair = it.pair0 + wave;
     const bool pair_live = pair * 64 < S.rows;
-    const bool two_tiles = pair * 64 + 32 < S.rows;          // the last pair may be one tile
     const int nf = pair_live ? (live + 15) / 16 : 0;         // live fragment columns, 0..4
-    const uint8_t * slot_base = A.bank + static_cast<size_t>(slot) * S.slot_bytes;
+    const uint8_t * slot_base = A.bank + static_cast<size_t>(it.slot) * S.slot_bytes;
 
     // weight stream: a buffer descriptor over the pair's codes (a dead pair reads the unit's first pair
     // and drops it; a missing second tile reads the first)
-    const int src_pair = pair_live ? pair : pair0;
+    const int src_pair = pair_live ? pair : it.pair0;
     const int tile1 = __builtin_amdgcn_readfirstlane(src_pair * 64 + 32 < S.rows ? 1 : 0);   // index of fragments 2, 3's tile
     const int code_tile = 32 * nb * 16, meta_tile = 32 * nb;
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
@@ -997,17 +434,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     // job's 512 bytes sits at part p ^ (job & 15), so that a fragment read (16 jobs, one part) covers
     // all banks. A load whose jobs are all past the tile's live ones is skipped; a dead job in a load
     // with a live one reads the tile's first job.
-    auto row_off16 = [&](int jl) __attribute__((always_inline)) -> uint32_t {               // row offset of live local job jl, in 16-byte units
-        const uint32_t jb = static_cast<uint32_t>(A.jobs[joff + j0 + jl]);
-        const uint32_t row = A.b_ne1 == 1 ? jb / static_cast<uint32_t>(A.n_ids) : jb;
-        return row * static_cast<uint32_t>(A.lay.stride() / 16);
-    };
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
     const int part = (lane & 31) ^ (2 * wave + (lane >> 5)); // of the loads with even i; odd i flip bit 3 (2k mod 16)
     const int djob = 32 * (wave & 1) + (lane >> 1);          // block scales: waves 0 and 1, 32 jobs x 32 bytes
     const uint8_t * da_base = A.rows_in + A.lay.da_offset();
     uint32_t * row_tab = reinterpret_cast<uint32_t *>(lds + L::OFF_ROW);
-    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
+    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
     __syncthreads();
     // (the rows' offsets are read back from LDS by every group: kept in registers they would spill, and
     // the spills' reloads wait for the DMA in flight)
@@ -1023,10 +455,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int k = wave + 4 * i;
-            if (2 * k < live) lds_dma_x4(base + static_cast<uint64_t>(row[i] + (i & 1 ? po : pe)) * 16, sb + k * 1024);
+            if (2 * k < live) lds_dma_x4(unit_ptr(base, row[i] + (i & 1 ? po : pe)), sb + k * 1024);
         }
         if (wave < 2 && 32 * wave < live)                    // (a tail of at most four blocks has no second 16 bytes)
-            lds_dma_x4(da_base + static_cast<uint64_t>(drow + 2 * g + (parts > 16 ? lane & 1 : 0)) * 16,
+            lds_dma_x4(unit_ptr(da_base, drow + 2 * g + (parts > 16 ? lane & 1 : 0)),
                        lds0 + (g & 1) * L::DA + wave * 1024);
     };
     // the wave's exponents of group g: lanes 0..15 / 16..31 bring the 256 bytes of its two tiles (the
@@ -1046,7 +478,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     if constexpr (FLAGGED) {
         int f = 0;
         if (lane < live)
-            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(lane)) * 16 + A.lay.flag_offset());
+            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(A, it, lane)) * 16 + A.lay.flag_offset());
         flagged = __any(f != 0);
     }
 
@@ -1226,86 +658,281 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     else if (nf == 3) k_loop(std::integral_constant<int, 3>{}, fold);
     else if (nf == 2) k_loop(std::integral_constant<int, 2>{}, fold);
     else k_loop(std::integral_constant<int, 1>{}, fold);
+    rows_epilogue<39, EPI>(A, it, pair, nf, acc);
+}
 
-    // Epilogue, from registers: lane (q, lr) holds rows 16i + 4q .. + 3 of the pair for job
-    // 16jh + lr. Biases (ggml row order), then fp32 rows (times the routing weight when given)
-    // as one 16-byte store per fragment, or GLU + Q8_0 requantization: fragments 0 / 1 and 2 / 3 are
-    // the gate / up rows of the block's elements 4q .. + 3 and 16 + 4q .. + 3.
-    float bias[4][4];
+// ------------------------------------------------------------------------- Q8_0 grouped GEMM
+// The same work split as the MXFP4 kernel above (64 rows x up to 64 jobs per wave, weights in registers,
+// activation stages of eight blocks in LDS) for int8 codes: a bank group is four blocks, so a stage is two
+// of them, each prefetched half a stage ahead. Block dots come from v_mfma_i32_16x16x32_i8, and the scale
+// products fp16(d_w) * d_act of four blocks of a 16 x 16 fragment from one v_mfma_f32_16x16x4_4b_f16, whose
+// four K = 4 blocks each hold one quantization block's scales at k = 0 and zeros: exact fp32 products of
+// two fp16 values, a quarter of a matrix instruction per block and nothing on the vector ALU, which is
+// left the int-to-float conversion and the FMA of every output and block.
+struct Q8StageLayout {
+    static constexpr int kJobs = 64;
+    static constexpr int ROW = 8 * 32;                         // int8 codes of a job and stage
+    static constexpr int DA = kJobs * 8 * 4;                   // [job][8 blocks] fp32 block scales, both stages first
+    static constexpr int OFF_ACT = 2 * DA, ACT = kJobs * ROW;
+    static constexpr int OFF_SC = OFF_ACT + 2 * ACT;           // [stage][wave][tile][group][32 rows] x 4 fp16
+    static constexpr int OFF_ROW = OFF_SC + 2 * 4 * 1024;      // [job] row offset in 16-byte units
+    static constexpr int BYTES = OFF_ROW + kJobs * 4;
+};
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int EPI, bool FLAGGED>
+__global__ __launch_bounds__(kGemmThreads, 2) void q8_rows_gemm_kernel(GemmArgs A) {
+    using L = Q8StageLayout;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[L::BYTES];
+    RowsItem it;
+    if (!rows_item<EPI>(A, L::kJobs, it)) return;
+    const GemmShape S = A.shape;
+    const int live = it.live;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int lr = lane & 15, q = lane >> 4;
+    const int nb = S.nb, stages = nb / 8, tail = nb % 8;      // full stages; blocks of a last partial one
+    const int n_stages = stages + (tail ? 1 : 0);
+    const int groups = nb / 4, n_groups = groups + (nb % 4 ? 1 : 0);   // a bank tail holds two blocks
+    const int pair = it.pair0 + wave;
+    const bool pair_live = pair * 64 < S.rows;
+    const int nf = pair_live ? (live + 15) / 16 : 0;         // live fragment columns, 0..4
+    const uint8_t * slot_base = A.bank + static_cast<size_t>(it.slot) * S.slot_bytes;
+
+    // weight stream, as in the MXFP4 kernel
+    const int src_pair = pair_live ? pair : it.pair0;
+    const int tile1 = __builtin_amdgcn_readfirstlane(src_pair * 64 + 32 < S.rows ? 1 : 0);   // index of fragments 2, 3's tile
+    const int code_tile = 32 * nb * 32, scale_tile = 32 * nb * 2;
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr(const_cast<uint8_t *>(slot_base + static_cast<size_t>(src_pair) * 2 * code_tile)), static_cast<short>(0),
+        __builtin_amdgcn_readfirstlane((1 + tile1) * code_tile), 0x00020000);
+    const uint8_t * scale_base = slot_base + S.codes_bytes + static_cast<size_t>(src_pair) * 2 * scale_tile;
+    auto load_group = [&](int g, MxGroupRegs & w) __attribute__((always_inline)) {
+        const int cs = g < groups ? 16 : 8;                  // bytes per (slice, row)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const bool row_live = i < 2 || two_tiles;
-        const int64_t grow = ggml_row(static_cast<int64_t>(pair) * 64 + 16 * i + 4 * q, S.rows, S.interleave);
+        for (int i = 0; i < 4; ++i) {
+            const int so = (i >> 1) * tile1 * code_tile + g * 4096;
+            w.c[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rc, (2 * q * 32 + 16 * (i & 1) + lr) * cs, so, 0);
+            w.c[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rc, ((2 * q + 1) * 32 + 16 * (i & 1) + lr) * cs, so, 0);
+        }
+    };
+    auto landed = [&](MxGroupRegs & w) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bias[i][j] = A.bias && row_live ? A.bias[static_cast<size_t>(expert) * S.rows + grow + j] : 0.0f;
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(w.c[i][0]), "+v"(w.c[i][1]));
+    };
+
+    // activation stages: DMA k = wave + 4i (1 KiB) holds jobs 4k..4k + 3; the 16-byte part p = 2b + q / 2 of a
+    // job's 256 bytes sits at part p ^ (job & 15)
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+    const int part = (lane & 15) ^ (4 * wave + (lane >> 4)); // 4k = 4 wave (mod 16): one part for every load
+    const int djob = 32 * (wave & 1) + (lane >> 1);          // block scales: waves 0 and 1, 32 jobs x 32 bytes
+    const uint8_t * da_base = A.rows_in + A.lay.da_offset();
+    uint32_t * row_tab = reinterpret_cast<uint32_t *>(lds + L::OFF_ROW);
+    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
+    __syncthreads();
+    auto dma_stage = [&](int s) __attribute__((always_inline)) {
+        const uint32_t sb = lds0 + L::OFF_ACT + (s & 1) * L::ACT;
+        const uint8_t * base = A.rows_in + static_cast<int64_t>(s) * L::ROW;
+        uint32_t row[4], drow = row_tab[djob];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) row[i] = row_tab[4 * (wave + 4 * i) + (lane >> 4)];
+        // the last stage: parts past its blocks read one of the first two blocks' again
+        const int parts = s < stages ? 16 : 2 * tail;
+        const uint32_t p = part < parts ? part : part & 3;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = wave + 4 * i;
+            if (4 * k < live) lds_dma_x4(unit_ptr(base, row[i] + p), sb + k * 1024);
+        }
+        if (wave < 2 && 32 * wave < live)                    // (a tail of at most four blocks has no second 16 bytes)
+            lds_dma_x4(unit_ptr(da_base, drow + 2 * s + (parts > 8 ? lane & 1 : 0)), lds0 + (s & 1) * L::DA + wave * 1024);
+    };
+    // the wave's weight scales of stage s: each half-wave brings the 512 bytes of one tile (the last
+    // stage's: 64 bytes per block)
+    auto dma_scales = [&](int s) __attribute__((always_inline)) {
+        if ((lane & 31) * 16 < 64 * (s < stages ? 8 : tail))
+            lds_dma_x4(scale_base + (lane >> 5) * tile1 * scale_tile + s * 512 + (lane & 31) * 16,
+                       lds0 + L::OFF_SC + ((s & 1) * 4 + wave) * 1024);
+    };
+
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jh = 0; jh < 4; ++jh) acc[i][jh] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bool flagged = false;                                    // wave-uniform: a live job holds -128 codes
+    if constexpr (FLAGGED) {
+        int f = 0;
+        if (lane < live)
+            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(A, it, lane)) * 16 + A.lay.flag_offset());
+        flagged = __any(f != 0);
     }
-    int jobs[4];
-    float scales[4];
+
+    // K loop over NF live fragment columns; GENERAL: with the exact -128 correction.
+    auto k_loop = [&](auto nf_c, auto general_c) __attribute__((always_inline)) {
+        constexpr int NF = decltype(nf_c)::value;
+        constexpr bool GENERAL = decltype(general_c)::value;
+        // this lane's 8 bytes of block 0 of fragment column 0; block b's are at the address with bits 5..7
+        // flipped by b
+        const uint32_t act0 = static_cast<uint32_t>(lr * L::ROW + (((q >> 1) ^ lr) << 4) + 8 * (q & 1));
+        // Bank group H of stage buffer st, its weights in w (nblk: 4, or the bank tail's 2, whose scales are
+        // packed by two per row).
+        auto half_stage = [&](int st, int H, const MxGroupRegs & w, int nblk, auto && issue) __attribute__((always_inline)) {
+            const uint8_t * sc_lds = lds + L::OFF_SC + (st * 4 + wave) * 1024 + H * 256;
+            const int srow = 2 * nblk;                       // scale bytes per row
+            const uint8_t * da_lds = lds + st * L::DA + 16 * H;
+            const uint8_t * act_lds = lds + L::OFF_ACT + st * L::ACT;
+            const uint32_t ah = act0 ^ (H << 7);
+            auto act = [&](int jh, int bb) __attribute__((always_inline)) {
+                return *reinterpret_cast<const long *>(act_lds + jh * 16 * L::ROW + (ah ^ (bb << 5)));
+            };
+            if constexpr (!GENERAL) {
+                half4_g as[4], bs[NF];                       // scales of block q of the group, at k = 0
+                unsigned dw[4];
+                float da[NF];
+                long bv[2][4];
 #pragma unroll
-    for (int jh = 0; jh < 4; ++jh) jobs[jh] = A.jobs[joff + j0 + (16 * jh + lr < live ? 16 * jh + lr : 0)];
+                for (int i = 0; i < 4; ++i) dw[i] = *reinterpret_cast<const uint16_t *>(sc_lds + (i >> 1) * 512 + (16 * (i & 1) + lr) * srow + 2 * q);
 #pragma unroll
-    for (int jh = 0; jh < 4; ++jh) scales[jh] = EPI == 0 && A.row_scale ? A.row_scale[jobs[jh]] : 1.0f;
+                for (int jh = 0; jh < NF; ++jh) da[jh] = *reinterpret_cast<const float *>(da_lds + (16 * jh + lr) * 32 + 4 * q);
 #pragma unroll
-    for (int jh = 0; jh < 4; ++jh) {
-        if (jh >= nf) break;
-        const bool jlive = 16 * jh + lr < live;
-        const int job = jobs[jh];
-        if constexpr (EPI == 0) {
-            const float rs = scales[jh];
+                for (int bb = 0; bb < 4; ++bb) bv[0][bb] = act(0, bb);
+                issue();
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (!jlive || (i >= 2 && !two_tiles)) continue;
-                float v[4];
+                for (int i = 0; i < 4; ++i) as[i] = __builtin_bit_cast(half4_g, u32x2g{dw[i], 0u});
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v[j] = acc[i][jh][j];
-                    if (A.bias) v[j] = v[j] + bias[i][j];
-                    if (A.row_scale) v[j] = v[j] * rs;
+                for (int jh = 0; jh < NF; ++jh)              // d_act holds fp16 values: exact
+                    bs[jh] = __builtin_bit_cast(half4_g, u32x2g{__builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(da[jh], 0.0f)), 0u});
+                // Software pipeline over the (column, fragment) steps: block bb's product of the previous step is
+                // scaled and summed right before its register takes this step's MFMA.
+                i32x4 d[4];
+                f32x16 sc[2];
+                auto sum = [&](int t, int bb) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[t % 4][t / 4][j] = __builtin_fmaf(sc[t & 1][4 * bb + j], static_cast<float>(d[bb][j]), acc[t % 4][t / 4][j]);
+                };
+#pragma unroll
+                for (int t = 0; t < 4 * NF; ++t) {
+                    const int i = t % 4, jh = t / 4;
+                    sc[t & 1] = __builtin_amdgcn_mfma_f32_16x16x4f16(as[i], bs[jh], f32x16{}, 0, 0, 0);
+                    if (i == 0 && jh + 1 < NF) {
+#pragma unroll
+                        for (int bb = 0; bb < 4; ++bb) bv[(jh + 1) & 1][bb] = act(jh + 1, bb);
+                    }
+#pragma unroll
+                    for (int bb = 0; bb < 4; ++bb) {
+                        if (bb >= 2 && nblk <= 2) break;
+                        if (t > 0) sum(t - 1, bb);
+                        const long a = static_cast<long>(static_cast<uint64_t>(w.c[i][0][bb]) | (static_cast<uint64_t>(w.c[i][1][bb]) << 32));
+                        d[bb] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bv[jh & 1][bb], i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    if (i == 0 && jh + 1 < NF) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+                    for (int bb = 0; bb < 4; ++bb) {
+                        if (t > 0) __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                // aligned runs of 4 device rows are 4 consecutive ggml rows, also in interleaved banks
-                float * out = A.dst + static_cast<size_t>(job) * S.rows +
-                              ggml_row(static_cast<int64_t>(pair) * 64 + 16 * i + 4 * q, S.rows, S.interleave);
-                if (A.dst_vec4) {
-                    *reinterpret_cast<float4 *>(out) = float4{v[0], v[1], v[2], v[3]};
-                } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) out[j] = v[j];
+                for (int bb = 0; bb < 4; ++bb)
+                    if (bb < 2 || nblk > 2) sum(4 * NF - 1, bb);
+                // keeps the sums in this place (see the MXFP4 kernel)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int jh = 0; jh < NF; ++jh) asm volatile("" : "+v"(acc[i][jh]));
+            } else {
+                issue();
+#pragma clang loop unroll(disable)
+                for (int bb = 0; bb < nblk; ++bb) {
+                    half8_t b16[NF];
+                    float da[NF];
+#pragma unroll
+                    for (int jh = 0; jh < NF; ++jh) {
+                        b16[jh] = i8_to_f16(act(jh, bb));
+                        da[jh] = *reinterpret_cast<const float *>(da_lds + (16 * jh + lr) * 32 + 4 * bb);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        auto pick = [&](const u32x4g & c) __attribute__((always_inline)) { return bb == 0 ? c[0] : (bb == 1 ? c[1] : (bb == 2 ? c[2] : c[3])); };
+                        const half8_t a16 = i8_to_f16(static_cast<long>(static_cast<uint64_t>(pick(w.c[i][0])) | (static_cast<uint64_t>(pick(w.c[i][1])) << 32)));
+                        float dw[4];                         // scales of output rows 16i + 4q + j
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            dw[j] = half_bits_to_float(*reinterpret_cast<const uint16_t *>(sc_lds + (i >> 1) * 512 + (16 * (i & 1) + 4 * q + j) * srow + 2 * bb));
+#pragma unroll
+                        for (int jh = 0; jh < NF; ++jh) {
+                            f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a16, b16[jh], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(neg_part(a16), is_neg128_x256(b16[jh]), d, 0, 0, 0);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) acc[i][jh][j] = __builtin_fmaf(dw[j] * da[jh], d[j], acc[i][jh][j]);
+                        }
+                    }
                 }
             }
-        } else {
-            float x[2][4], amax = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float gv = acc[2 * t][jh][j], uv = acc[2 * t + 1][jh][j];
-                    if (A.bias) gv = gv + bias[2 * t][j], uv = uv + bias[2 * t + 1][j];
-                    x[t][j] = glu_fast(A.activation, gv, uv, A.alpha, A.limit);
-                    amax = fmaxf(amax, fabsf(x[t][j]));
+        };
+        MxGroupRegs wa, wb;
+        load_group(0, wa);
+        lds_dma_wait<0>();
+        landed(wa);
+        __syncthreads();
+#pragma clang loop unroll(disable)
+        for (int s = 0; s < stages; ++s) {
+            const int st = s & 1;
+            half_stage(st, 0, wa, 4, [&]() __attribute__((always_inline)) {
+                if (s + 1 < n_stages) {
+                    dma_stage(s + 1);
+                    dma_scales(s + 1);
                 }
-            amax = fmaxf(amax, __shfl_xor(amax, 16));        // the block's other lanes of this job
-            amax = fmaxf(amax, __shfl_xor(amax, 32));
-            const float d = amax / 127.0f;
-            const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
-            if (!jlive) continue;
-            uint8_t * out = A.rows_out + static_cast<int64_t>(job) * A.out_lay.stride();
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                half4_g c;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float v = rintf(x[t][j] * id);
-                    v = v > 127.0f ? 127.0f : (v < -128.0f ? -128.0f : v);
-                    c[j] = static_cast<_Float16>(v);
-                }
-                *reinterpret_cast<half4_g *>(out + (static_cast<int64_t>(pair) * 32 + 16 * t + 4 * q) * 2) = c;
-            }
-            if (q == 0) {
-                reinterpret_cast<float *>(out + A.out_lay.da_offset())[pair] = static_cast<float>(static_cast<_Float16>(d));
-                if (pair == 0) *reinterpret_cast<int *>(out + A.out_lay.flag_offset()) = 0;   // never -128
+                load_group(2 * s + 1, wb);
+            });
+            half_stage(st, 1, wb, 4, [&]() __attribute__((always_inline)) {
+                load_group(__builtin_amdgcn_readfirstlane(2 * s + 2 < n_groups ? 2 * s + 2 : n_groups - 1), wa);
+            });
+            lds_dma_wait<0>();
+            landed(wa);
+            __syncthreads();
+        }
+        if (tail) {   // 2, 4 or 6 blocks: a bank tail, a group, or both
+            const int st = stages & 1;
+            if (tail == 2) {
+                half_stage(st, 0, wa, 2, [] {});
+            } else {
+                half_stage(st, 0, wa, 4, [&]() __attribute__((always_inline)) { load_group(n_groups - 1, wb); });
+                if (tail == 6) half_stage(st, 1, wb, 2, [] {});
             }
         }
+    };
+    dma_stage(0);
+    dma_scales(0);
+    // Waves may take different instantiations: each issues the same stage loads and reaches the same
+    // number of barriers.
+    if (nf == 0) {
+        lds_dma_wait<0>();
+        __syncthreads();
+        for (int s = 1; s < n_stages; ++s) {
+            dma_stage(s);
+            lds_dma_wait<0>();
+            __syncthreads();
+        }
+        if (!tail) __syncthreads();
+        return;
     }
+    constexpr std::false_type fast{};
+    if constexpr (FLAGGED) {
+        if (flagged) {
+            k_loop(std::integral_constant<int, 4>{}, std::true_type{});
+            rows_epilogue<8, EPI>(A, it, pair, nf, acc);
+            return;
+        }
+    }
+    if (nf == 4) k_loop(std::integral_constant<int, 4>{}, fast);
+    else if (nf == 3) k_loop(std::integral_constant<int, 3>{}, fast);
+    else if (nf == 2) k_loop(std::integral_constant<int, 2>{}, fast);
+    else k_loop(std::integral_constant<int, 1>{}, fast);
+    rows_epilogue<8, EPI>(A, it, pair, nf, acc);
 }
 
 // Tiles of job_tile jobs per active expert, in active order: one workgroup, wave scans plus a
@@ -1448,23 +1075,14 @@ __global__ __launch_bounds__(256) void gemm_rows_from_q8_kernel(const uint8_t * 
     if (threadIdx.x == 0) *reinterpret_cast<int *>(o + L.flag_offset()) = s_flag;
 }
 
-template <int EPI, bool FLAGGED>
-void launch_mx_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
+template <int TYPE, int EPI, bool FLAGGED>
+void launch_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
     GemmArgs b = a;
     b.row_units = static_cast<int>((rows + 255) / 256);
     const int64_t items = static_cast<int64_t>(b.row_units) * max_tiles;
-    hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)), dim3(kGemmThreads), 0,
-                       stream, b);
-    check_hip(hipGetLastError(), "grouped GEMM launch");
-}
-
-template <int TYPE, int EPI, bool FLAGGED>
-void launch_gemm_typed(const GemmArgs & a, int row_pairs, int max_tiles, hipStream_t stream) {
-    GemmArgs b = a;
-    b.row_pairs = row_pairs;
-    const int64_t items = static_cast<int64_t>(row_pairs) * max_tiles;
-    hipLaunchKernelGGL((grouped_gemm_kernel<TYPE, EPI, FLAGGED>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)),
-                       dim3(kGemmThreads), 0, stream, b);
+    const dim3 grid(static_cast<unsigned>((items + 7) / 8 * 8));
+    if constexpr (TYPE == 39) hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
+    else hipLaunchKernelGGL((q8_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
     check_hip(hipGetLastError(), "grouped GEMM launch");
 }
 
@@ -1830,20 +1448,19 @@ void launch_grouped_gemm(const GemmParams & p, hipStream_t stream) {
     a.activation = p.activation;
     a.alpha = p.alpha;
     a.limit = p.limit;
-    const int row_pairs = static_cast<int>((bank.rows + 63) / 64);
     require(!p.flagged_rows || p.epilogue == 0, "flagged activation rows only with the plain epilogue");
     // the launch covers max_tiles tiles, or the caller's bound on this call's tiles (its tile filter
     // leaves only the experts whose tiles it counted)
     require(p.grid_tiles >= 0 && (p.grid_tiles == 0 || p.tile_filter != nullptr), "grid tile bound needs a tile filter");
     const int mt = static_cast<int>(p.grid_tiles > 0 ? std::min<int64_t>(p.grid_tiles, max_tiles) : max_tiles);
     if (bank.type == VBM_TYPE_MXFP4) {
-        if (p.flagged_rows) launch_mx_rows_gemm<0, true>(a, bank.rows, mt, stream);
-        else if (p.epilogue == 0) launch_mx_rows_gemm<0, false>(a, bank.rows, mt, stream);
-        else launch_mx_rows_gemm<1, false>(a, bank.rows, mt, stream);
+        if (p.flagged_rows) launch_rows_gemm<39, 0, true>(a, bank.rows, mt, stream);
+        else if (p.epilogue == 0) launch_rows_gemm<39, 0, false>(a, bank.rows, mt, stream);
+        else launch_rows_gemm<39, 1, false>(a, bank.rows, mt, stream);
     } else {
-        if (p.flagged_rows) launch_gemm_typed<8, 0, true>(a, row_pairs, mt, stream);
-        else if (p.epilogue == 0) launch_gemm_typed<8, 0, false>(a, row_pairs, mt, stream);
-        else launch_gemm_typed<8, 1, false>(a, row_pairs, mt, stream);
+        if (p.flagged_rows) launch_rows_gemm<8, 0, true>(a, bank.rows, mt, stream);
+        else if (p.epilogue == 0) launch_rows_gemm<8, 0, false>(a, bank.rows, mt, stream);
+        else launch_rows_gemm<8, 1, false>(a, bank.rows, mt, stream);
     }
 }
 

@@ -237,10 +237,8 @@ struct GemmParams {
     int64_t grid_tiles;               // > 0: bound on the tiles left by tile_filter (launch size), else 0
     bool tiles_ready;                 // `tiles` already holds this group's list (same group and filter)
 };
-// Jobs per grouped-GEMM workgroup (one expert's job tile): 192 for Q8_0 banks, whose expert groups
-// at 2048 tokens top-8 over 128 experts hold 96-158 jobs (one tile each instead of a nearly empty
-// second tile for half of them), 64 for MXFP4 (a wave's 4 x 4 fragments).
-inline int gemm_job_tile(int bank_type) { return bank_type == VBM_TYPE_MXFP4 ? 64 : 192; }
+// Jobs per grouped-GEMM workgroup (one expert's job tile): a wave's four 16-job fragment columns.
+inline int gemm_job_tile(int) { return 64; }
 int64_t gemm_max_tiles(int64_t n_as, int64_t n_entries, int job_tile);
 size_t gemm_tiles_bytes(int64_t n_as, int64_t n_entries);
 void launch_grouped_gemm(const GemmParams & p, hipStream_t stream);
