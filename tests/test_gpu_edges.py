@@ -75,3 +75,31 @@ def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, exp
         got = out.download(np.float32, (1, hidden))
         assert H.bits_equal(got, ref["out"]), H.diff_report(got, ref["out"])
     layer.destroy()
+
+
+@pytest.mark.parametrize("top_k,hidden", [(1, 320), (8, 256), (9, 320), (17, 64)])
+def test_decode_step_finish_matches_layer_calls(gpu, top_k, hidden):
+    """The step's last launch combines the ranks in batches of eight and hands out ids and weights: two
+    chained layers against two one-token layer calls, bit for bit, with and without the optional outputs."""
+    experts, inter, L = 20, 128, 2
+    layers = [Layer(gpu, H.MX, hidden, inter, experts, top_k, seed=33, layer=l, router=False) for l in range(L)]
+    x = gpu.synth_normal(33, 6, 0, hidden).reshape(1, hidden)
+    logits = gpu.synth_normal(33, 7, 0, L * experts).reshape(L, experts)
+    want, want_ids, want_w = x, [], []
+    for l in range(L):
+        want, i, w = layers[l].forward_gpu(want, logits[l:l + 1])
+        want_ids.append(i), want_w.append(w)
+    plan = C.c_void_p()
+    gpu.call("vbm_decode_plan_create", (gpu.MoeLayerDesc * L)(*[l.desc() for l in layers]), L, C.byref(plan))
+    dx, dl = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer.from_array(logits)
+    for outputs in (True, False):
+        out, ids, w = gpu.DeviceBuffer(4 * hidden), gpu.DeviceBuffer(4 * L * top_k), gpu.DeviceBuffer(4 * L * top_k)
+        gpu.call("vbm_decode_step", plan.value, dx.ptr, dl.ptr, out.ptr, ids.ptr if outputs else None, w.ptr if outputs else None, None, None)
+        gpu.call("vbm_stream_synchronize", None)
+        assert H.bits_equal(out.download(np.float32, (1, hidden)), want)
+        if outputs:
+            assert np.array_equal(ids.download(np.int32, (L, top_k)), np.concatenate(want_ids))
+            assert H.bits_equal(w.download(np.float32, (L, top_k)), np.concatenate(want_w))
+    gpu.call("vbm_decode_plan_destroy", plan.value)
+    for l in layers:
+        l.destroy()

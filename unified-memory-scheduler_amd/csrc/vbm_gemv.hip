@@ -197,11 +197,12 @@ __device__ __forceinline__ void q8_group(const u32x4 & c, const u32x2 & m, int b
 
 // Weight groups a lane keeps in flight. Both MXFP4 decode kernels stream through a 5-deep ring
 // so compute overlaps the arrivals (120B-shape decode, A / B depth 6 / 12: 1511-1514 tok/s, 5 / 6:
-// 1600-1618, 5 / 5: 1627-1638, 6 / 4: 1540-1561, 7 / 6: 1522-1531); the batched kernel's depth is
-// set where it streams (gemv_chunk).
+// 1600-1618, 5 / 5: 1627-1638, 6 / 4: 1540-1561, 7 / 6: 1522-1531); Q8_0 through an 8-deep one (three layers of
+// hidden 2048, inter 768, top-8: depth 4 50.3 us, 6 50.1, 8 49.2, 16 51.0). The batched kernel's depth
+// is set where it streams (gemv_chunk).
 template <int TYPE>
 constexpr int gate_up_depth() {
-    return TYPE == 39 ? 5 : 4;
+    return TYPE == 39 ? 5 : 8;
 }
 template <int TYPE>
 constexpr int down_depth() {

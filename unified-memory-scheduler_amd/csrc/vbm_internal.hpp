@@ -127,6 +127,10 @@ void launch_router(const float * router_w, const float * router_b, const float *
 // NULL: the rows are already weighted, out[t] = sum of y[t][r] in rank order.
 void launch_combine(const float * y, const float * weights, int64_t rows, int64_t n_ids, int64_t n_tokens,
                     float * out, hipStream_t stream);
+// A decode step's last launch: launch_combine of one token (weighted), and n_routes ids / weights copied to
+// ids_out / weights_out (device memory, or null).
+void launch_decode_finish(const float * y, const float * w, int64_t rows, int64_t n_ids, float * out, const int32_t * ids,
+                          int32_t * ids_out, const float * weights, float * weights_out, int64_t n_routes, hipStream_t stream);
 void launch_glu(int activation, const float * gate, const float * up, float * out, int64_t n_rows,
                 int64_t width, int64_t gate_stride, int64_t up_stride, int64_t out_stride, float alpha,
                 float limit, hipStream_t stream);

@@ -734,6 +734,18 @@ vbm_status vbm_decode_plan_destroy(vbm_decode_plan * plan) {
 
 namespace {
 
+// 4-byte aligned memory of the plan's device (a kernel may write it).
+bool on_device(const void * p) {
+    if (p == nullptr || reinterpret_cast<uintptr_t>(p) % 4 != 0) return false;
+    hipPointerAttribute_t attr{};
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int device = 0;
+    return attr.type == hipMemoryTypeDevice && hipGetDevice(&device) == hipSuccess && attr.device == device;
+}
+
 void decode_launch_a(const vbm_decode_plan * plan, int64_t l, const float * x, const float * logits, hipStream_t s) {
     const vbm_moe_layer_desc & d = plan->layers[l];
     const int64_t K = plan->K;
@@ -875,9 +887,14 @@ vbm_status vbm_decode_step(vbm_decode_plan * plan, const float * x, const float 
             decode_launch_b(plan, l, s);
             record(ev, 3, s);
         }
-        launch_combine(plan->y, plan->route_w + (plan->L - 1) * K, H, K, 1, out, s);
-        if (ids) check_hip(hipMemcpyAsync(ids, plan->route_ids, sizeof(int32_t) * plan->L * K, hipMemcpyDeviceToDevice, s), "ids copy");
-        if (weights) check_hip(hipMemcpyAsync(weights, plan->route_w, sizeof(float) * plan->L * K, hipMemcpyDeviceToDevice, s), "weights copy");
+        // the routing leaves with the combine when its buffers are device memory (any other memory the
+        // runtime can copy to keeps the copies)
+        int32_t * ids_dev = on_device(ids) ? ids : nullptr;
+        float * weights_dev = on_device(weights) ? weights : nullptr;
+        launch_decode_finish(plan->y, plan->route_w + (plan->L - 1) * K, H, K, out, plan->route_ids, ids_dev, plan->route_w,
+                             weights_dev, plan->L * K, s);
+        if (ids && !ids_dev) check_hip(hipMemcpyAsync(ids, plan->route_ids, sizeof(int32_t) * plan->L * K, hipMemcpyDeviceToDevice, s), "ids copy");
+        if (weights && !weights_dev) check_hip(hipMemcpyAsync(weights, plan->route_w, sizeof(float) * plan->L * K, hipMemcpyDeviceToDevice, s), "weights copy");
     });
 }
 

@@ -421,6 +421,41 @@ __global__ void combine_kernel(const float * __restrict__ y, const float * __res
     out[idx] = acc;
 }
 
+// The end of a decode step in one launch: the last layer's rank combine (the first combine_blocks
+// workgroups, one row per thread, every rank's load in flight together) and the step's routing copied to the
+// caller's buffers (the others; null destinations are skipped). As two copies behind the combine they cost
+// a launch and a barrier each (three Q8_0 layers launched eagerly: 49.2 -> 46.6 us).
+__global__ __launch_bounds__(256) void decode_finish_kernel(const float * __restrict__ y, const float * __restrict__ w, int rows,
+                                                            int n_ids, float * __restrict__ out, int combine_blocks,
+                                                            const int32_t * __restrict__ ids, int32_t * __restrict__ ids_out,
+                                                            const float * __restrict__ weights, float * __restrict__ weights_out,
+                                                            int n_routes) {
+    const int b = static_cast<int>(blockIdx.x);
+    if (b >= combine_blocks) {
+        const int i = (b - combine_blocks) * 256 + static_cast<int>(threadIdx.x);
+        if (i < n_routes) {
+            if (ids_out) ids_out[i] = ids[i];
+            if (weights_out) weights_out[i] = weights[i];
+        }
+        return;
+    }
+    const int i = b * 256 + static_cast<int>(threadIdx.x);
+    if (i >= rows) return;
+    float acc = 0.0f;
+    for (int r0 = 0; r0 < n_ids; r0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = r0 + j < n_ids ? y[static_cast<int64_t>(r0 + j) * rows + i] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (r0 + j < n_ids) {
+                const float term = v[j] * w[r0 + j];
+                acc = r0 + j == 0 ? term : acc + term;
+            }
+    }
+    out[i] = acc;
+}
+
 __global__ void glu_kernel(int activation, const float * __restrict__ gate, const float * __restrict__ up,
                            float * __restrict__ out, int64_t n_rows, int64_t width, int64_t gs, int64_t us,
                            int64_t os, float alpha, float limit) {
@@ -656,6 +691,15 @@ void launch_combine(const float * y, const float * weights, int64_t rows, int64_
                            dim3(256), 0, stream, y, weights, rows, static_cast<int>(n_ids), n_tokens, out);
     }
     check_hip(hipGetLastError(), "combine launch");
+}
+
+void launch_decode_finish(const float * y, const float * w, int64_t rows, int64_t n_ids, float * out, const int32_t * ids,
+                          int32_t * ids_out, const float * weights, float * weights_out, int64_t n_routes, hipStream_t stream) {
+    require(rows > 0 && rows < (1ll << 30) && n_ids > 0 && n_routes >= 0 && n_routes < (1ll << 30), "decode finish shape out of range");
+    const unsigned cb = blocks_for(rows, 256), rb = ids_out || weights_out ? blocks_for(n_routes, 256) : 0;
+    hipLaunchKernelGGL(decode_finish_kernel, dim3(cb + rb), dim3(256), 0, stream, y, w, static_cast<int>(rows), static_cast<int>(n_ids),
+                       out, static_cast<int>(cb), ids, ids_out, weights, weights_out, static_cast<int>(n_routes));
+    check_hip(hipGetLastError(), "decode finish launch");
 }
 
 void launch_glu(int activation, const float * gate, const float * up, float * out, int64_t n_rows, int64_t width,
