@@ -85,6 +85,19 @@ __device__ __forceinline__ float dpp_move(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// 2^(b - 127) for byte N of `w`, b its value: the byte in the f32 exponent field, one instruction by byte
+// select (the compiler takes a shift and a mask for bytes 0..2).
+template <int N>
+__device__ __forceinline__ float exp2_byte(unsigned w) {
+    float r;
+    const unsigned shift = 23;
+    if constexpr (N == 0) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "v"(shift), "v"(w));
+    else if constexpr (N == 1) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "v"(shift), "v"(w));
+    else if constexpr (N == 2) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "v"(shift), "v"(w));
+    else asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "v"(shift), "v"(w));
+    return r;
+}
+
 // Maximum over each aligned group of four lanes (all four active).
 __device__ __forceinline__ float quad_max(float v) {
     v = fmaxf(v, dpp_move<0xB1>(v));

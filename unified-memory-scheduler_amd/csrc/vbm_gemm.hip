@@ -521,7 +521,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) ew[i] ^= 0x80808080u;
                 auto weights = [&](int i, int bb) __attribute__((always_inline)) {
-                    const float sc = __builtin_bit_cast(float, ((ew[i] >> (8 * bb)) & 0xFFu) << 23);   // 2^(e+1)
+                    const float sc = bb == 0 ? exp2_byte<0>(ew[i]) : (bb == 1 ? exp2_byte<1>(ew[i]) : (bb == 2 ? exp2_byte<2>(ew[i]) : exp2_byte<3>(ew[i])));   // 2^(e+1)
                     return mx_a_operand(w.c[i][0][2 * H + (bb >> 1)], w.c[i][1][2 * H + (bb >> 1)], bb & 1, sc);
                 };
                 // Software pipeline over the (block, column) steps: fragment i's product of the previous

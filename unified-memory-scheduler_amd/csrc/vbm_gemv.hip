@@ -475,11 +475,9 @@ __device__ __forceinline__ void group_mm(const u32x4 & c, const u32x2 & m, const
         auto pair = [&](auto q_c) __attribute__((always_inline)) {
             constexpr int Q = decltype(q_c)::value;
             const unsigned r = Q < 2 ? r0 : r1, s = Q < 2 ? m.x : m.y;
-            constexpr int B0 = 16 * (Q & 1), B1 = B0 + 8;
-            mx_block_mm<M, 0, 0, N0 + 2 * Q, FOLD>(c[Q], __builtin_bit_cast(float, ((r >> B0) & 0xFFu) << 23),
-                                                   static_cast<signed char>(s >> B0), act, acc);
-            mx_block_mm<M, 2, 1, N0 + 2 * Q + 1, FOLD>(c[Q], __builtin_bit_cast(float, ((r >> B1) & 0xFFu) << 23),
-                                                       static_cast<signed char>(s >> B1), act, acc);
+            constexpr int B0 = 2 * (Q & 1), B1 = B0 + 1;
+            mx_block_mm<M, 0, 0, N0 + 2 * Q, FOLD>(c[Q], FOLD ? exp2_byte<B0>(r) : 0.0f, static_cast<signed char>(s >> (8 * B0)), act, acc);
+            mx_block_mm<M, 2, 1, N0 + 2 * Q + 1, FOLD>(c[Q], FOLD ? exp2_byte<B1>(r) : 0.0f, static_cast<signed char>(s >> (8 * B1)), act, acc);
             __builtin_amdgcn_sched_barrier(0);
         };
         pair(std::integral_constant<int, 0>{});
