@@ -59,7 +59,7 @@ enum {
  *   VBM_ORDER_FAST: per-block integer dots are still exact; the fp32 accumulation order is free,
  *     and a fused layer's GLU (gate_up GEMM epilogue) uses a fast exp and divide.
  *     Calls of >= 16 tokens with >= 12 routed rows per expert on average run the MFMA grouped GEMM;
- *     the others run the exact-order GEMV (faster there, and its results satisfy either order). */
+ *     the others run the exact-order GEMV, with the exact order's bits. */
 enum { VBM_ORDER_EXACT = 0, VBM_ORDER_FAST = 1 };
 
 const char * vbm_last_error(void);

@@ -268,10 +268,11 @@ struct LayerWorkspace {
     size_t total;
 };
 constexpr int64_t kGemmMinTokens = 16;
-// Below 12 routed rows per expert on average the exact-order batched GEMV (matrix-core slice
-// dots, one workgroup per job chunk) outruns the MFMA grouped GEMM: 6-layer stacks of the
-// 2880 x 2880 MXFP4 shape, top-4, 32 / 128 experts, GEMV vs GEMM tok/s at 8 rows 47.6k vs 38.6k /
-// 56.8k vs 44.6k, at 12 rows 54.8k vs 56.4k / 62.0k vs 64.7k, at 16 rows 60.4k vs 72.4k.
+// Below 12 routed rows per expert on average a fast-order call keeps the exact-order batched GEMV, and
+// with it the exact order's bits, which the interface states. The line is that promise, not the
+// crossover any more: one layer of the 2880 x 2880 MXFP4 shape, top-4, 32 / 128 experts, GEMV against
+// GEMM: 2 rows 103 / 111 and 336 / 308 us, 4 rows 128 / 113 and 443 / 358 us, 8 rows 180 / 115 and 638 / 371 us, 12
+// rows 233 / 125 and 846 / 386 us.
 constexpr int64_t kGemmMinRowsPerExpert = 12;
 bool use_gemm(const vbm_moe_layer_desc & d, int64_t n_tokens);
 inline bool gemm_pays(int64_t n_tokens, int64_t top_k, int64_t n_expert) {
