@@ -64,6 +64,14 @@ def test_bank_layout_bijection_host(tmp_path):
     assert "bijective" in proc.stdout
 
 
+def test_gemm_row_addresses_host(tmp_path):
+    exe = tmp_path / "test_gemm_rows"
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{REPO / 'unified-memory-scheduler_amd' / 'csrc'}",
+                    str(REPO / "tests" / "cpp" / "test_gemm_rows.cpp"), "-o", str(exe)], check=True)
+    proc = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
 @pytest.mark.parametrize("args,needle", [(["--gpus", "2"], "exactly one GPU"), (["--tokens", "4"], "single-token")])
 def test_bench_refuses_unsupported_runs(args, needle):
     """bench.py measures one GPU at batch 1: other requests exit with status 2 and a message,

@@ -218,4 +218,17 @@ VBM_HD void q8_load_block(const uint8_t * slot, const SlotGeometry & g, int64_t 
     blk[0] = slot[s]; blk[1] = slot[s + 1];
 }
 
+// Activation row of the MFMA grouped GEMM: row-major codes (f16 for MXFP4 weights, int8 for
+// Q8_0), fp16-rounded fp32 block scales, and the row's -128 flag; 256-byte aligned stride.
+struct GemmRowLayout {
+    int64_t nb;
+    int weight_type;
+    VBM_HD int64_t code_bytes() const { return nb * 32 * (weight_type == 39 ? 2 : 1); }
+    VBM_HD int64_t da_offset() const { return code_bytes(); }
+    VBM_HD int64_t flag_offset() const { return da_offset() + 4 * nb; }
+    VBM_HD int64_t stride() const { return (flag_offset() + 4 + 255) / 256 * 256; }
+    // Byte offset of a row: the rows that a launch admits go past 64 GiB.
+    VBM_HD uint64_t row_offset(uint32_t row) const { return static_cast<uint64_t>(row) * static_cast<uint64_t>(stride()); }
+};
+
 }  // namespace vbm

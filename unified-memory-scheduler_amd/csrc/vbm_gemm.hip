@@ -209,8 +209,8 @@ struct MxStageLayout {
     static constexpr int DA = kJobs * 8 * 4;                   // [job][8 blocks] fp32 block scales, both stages first
     static constexpr int OFF_ACT = 2 * DA, ACT = kJobs * ROW;  // (every fragment read then has a 16-bit offset)
     static constexpr int OFF_EXP = OFF_ACT + 2 * ACT;          // [stage][wave][64 rows] x 8 exponent bytes
-    static constexpr int OFF_ROW = OFF_EXP + 2 * 4 * 512;      // [job] row offset in 16-byte units
-    static constexpr int BYTES = OFF_ROW + kJobs * 4;
+    static constexpr int OFF_ROW = OFF_EXP + 2 * 4 * 512;      // [job] address of the row
+    static constexpr int BYTES = OFF_ROW + kJobs * 8;
 };
 // Weights of a wave and group: entry [i][s] is slice 2q + s of row 16i + lr (dword d holds blocks
 // 2d, 2d + 1). Their exponents are staged in LDS: as registers too they would spill.
@@ -267,14 +267,10 @@ __device__ __forceinline__ bool rows_item(const GemmArgs & A, int job_tile, Rows
     return false;
 }
 
-// Byte address of 16-byte unit `off` of `base`.
-__device__ __forceinline__ const uint8_t * unit_ptr(const uint8_t * base, uint32_t off) { return base + static_cast<uint64_t>(off) * 16; }
-
-// Row offset of live local job jl, in 16-byte units.
-__device__ __forceinline__ uint32_t row_off16(const GemmArgs & A, const RowsItem & it, int jl) {
+// Activation row of live local job jl.
+__device__ __forceinline__ const uint8_t * job_row(const GemmArgs & A, const RowsItem & it, int jl) {
     const uint32_t jb = static_cast<uint32_t>(A.jobs[it.joff + it.j0 + jl]);
-    const uint32_t row = A.b_ne1 == 1 ? jb / static_cast<uint32_t>(A.n_ids) : jb;
-    return row * static_cast<uint32_t>(A.lay.stride() / 16);
+    return A.rows_in + A.lay.row_offset(A.b_ne1 == 1 ? jb / static_cast<uint32_t>(A.n_ids) : jb);
 }
 
 // Epilogue, from registers: lane (q, lr) holds rows 16i + 4q .. + 3 of tile pair `pair` for job 16jh + lr, jh < nf.
@@ -438,28 +434,28 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
     const int part = (lane & 31) ^ (2 * wave + (lane >> 5)); // of the loads with even i; odd i flip bit 3 (2k mod 16)
     const int djob = 32 * (wave & 1) + (lane >> 1);          // block scales: waves 0 and 1, 32 jobs x 32 bytes
-    const uint8_t * da_base = A.rows_in + A.lay.da_offset();
-    uint32_t * row_tab = reinterpret_cast<uint32_t *>(lds + L::OFF_ROW);
-    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
+    const uint32_t da_off = static_cast<uint32_t>(A.lay.da_offset());
+    const uint8_t ** row_tab = reinterpret_cast<const uint8_t **>(lds + L::OFF_ROW);
+    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = job_row(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
     __syncthreads();
-    // (the rows' offsets are read back from LDS by every group: kept in registers they would spill, and
+    // (the rows' addresses are read back from LDS by every group: kept in registers they would spill, and
     // the spills' reloads wait for the DMA in flight)
     auto dma_stage = [&](int g) __attribute__((always_inline)) {
         const uint32_t sb = lds0 + L::OFF_ACT + (g & 1) * L::ACT;
-        const uint8_t * base = A.rows_in + static_cast<int64_t>(g) * L::ROW;
-        uint32_t row[8], drow = row_tab[djob];
+        const uint8_t * row[8], * drow = row_tab[djob];
 #pragma unroll
         for (int i = 0; i < 8; ++i) row[i] = row_tab[2 * (wave + 4 * i) + (lane >> 5)];
         // the tail's stage: parts past its blocks read one of the first two blocks' again
         const int parts = g < groups ? 32 : 4 * tail;
-        const uint32_t pe = part < parts ? part : part & 7, po = (part ^ 8) < parts ? part ^ 8 : part & 7;
+        const uint32_t pe = g * L::ROW + 16 * (part < parts ? part : part & 7);
+        const uint32_t po = g * L::ROW + 16 * ((part ^ 8) < parts ? part ^ 8 : part & 7);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int k = wave + 4 * i;
-            if (2 * k < live) lds_dma_x4(unit_ptr(base, row[i] + (i & 1 ? po : pe)), sb + k * 1024);
+            if (2 * k < live) lds_dma_x4(row[i] + (i & 1 ? po : pe), sb + k * 1024);
         }
         if (wave < 2 && 32 * wave < live)                    // (a tail of at most four blocks has no second 16 bytes)
-            lds_dma_x4(unit_ptr(da_base, drow + 2 * g + (parts > 16 ? lane & 1 : 0)),
+            lds_dma_x4(drow + (da_off + 16 * (2 * g + (parts > 16 ? lane & 1 : 0))),
                        lds0 + (g & 1) * L::DA + wave * 1024);
     };
     // the wave's exponents of group g: lanes 0..15 / 16..31 bring the 256 bytes of its two tiles (the
@@ -479,7 +475,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
     if constexpr (FLAGGED) {
         int f = 0;
         if (lane < live)
-            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(A, it, lane)) * 16 + A.lay.flag_offset());
+            f = *reinterpret_cast<const int *>(job_row(A, it, lane) + A.lay.flag_offset());
         flagged = __any(f != 0);
     }
 
@@ -677,8 +673,8 @@ struct Q8StageLayout {
     static constexpr int DA = kJobs * 8 * 4;                   // [job][8 blocks] fp32 block scales, both stages first
     static constexpr int OFF_ACT = 2 * DA, ACT = kJobs * ROW;
     static constexpr int OFF_SC = OFF_ACT + 2 * ACT;           // [stage][wave][tile][group][32 rows] x 4 fp16
-    static constexpr int OFF_ROW = OFF_SC + 2 * 4 * 1024;      // [job] row offset in 16-byte units
-    static constexpr int BYTES = OFF_ROW + kJobs * 4;
+    static constexpr int OFF_ROW = OFF_SC + 2 * 4 * 1024;      // [job] address of the row
+    static constexpr int BYTES = OFF_ROW + kJobs * 8;
 };
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -727,26 +723,25 @@ __global__ __launch_bounds__(kGemmThreads, 2) void q8_rows_gemm_kernel(GemmArgs 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
     const int part = (lane & 15) ^ (4 * wave + (lane >> 4)); // 4k = 4 wave (mod 16): one part for every load
     const int djob = 32 * (wave & 1) + (lane >> 1);          // block scales: waves 0 and 1, 32 jobs x 32 bytes
-    const uint8_t * da_base = A.rows_in + A.lay.da_offset();
-    uint32_t * row_tab = reinterpret_cast<uint32_t *>(lds + L::OFF_ROW);
-    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = row_off16(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
+    const uint32_t da_off = static_cast<uint32_t>(A.lay.da_offset());
+    const uint8_t ** row_tab = reinterpret_cast<const uint8_t **>(lds + L::OFF_ROW);
+    if (threadIdx.x < L::kJobs) row_tab[threadIdx.x] = job_row(A, it, static_cast<int>(threadIdx.x) < live ? static_cast<int>(threadIdx.x) : 0);
     __syncthreads();
     auto dma_stage = [&](int s) __attribute__((always_inline)) {
         const uint32_t sb = lds0 + L::OFF_ACT + (s & 1) * L::ACT;
-        const uint8_t * base = A.rows_in + static_cast<int64_t>(s) * L::ROW;
-        uint32_t row[4], drow = row_tab[djob];
+        const uint8_t * row[4], * drow = row_tab[djob];
 #pragma unroll
         for (int i = 0; i < 4; ++i) row[i] = row_tab[4 * (wave + 4 * i) + (lane >> 4)];
         // the last stage: parts past its blocks read one of the first two blocks' again
         const int parts = s < stages ? 16 : 2 * tail;
-        const uint32_t p = part < parts ? part : part & 3;
+        const uint32_t p = s * L::ROW + 16 * (part < parts ? part : part & 3);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int k = wave + 4 * i;
-            if (4 * k < live) lds_dma_x4(unit_ptr(base, row[i] + p), sb + k * 1024);
+            if (4 * k < live) lds_dma_x4(row[i] + p, sb + k * 1024);
         }
         if (wave < 2 && 32 * wave < live)                    // (a tail of at most four blocks has no second 16 bytes)
-            lds_dma_x4(unit_ptr(da_base, drow + 2 * s + (parts > 8 ? lane & 1 : 0)), lds0 + (s & 1) * L::DA + wave * 1024);
+            lds_dma_x4(drow + (da_off + 16 * (2 * s + (parts > 8 ? lane & 1 : 0))), lds0 + (s & 1) * L::DA + wave * 1024);
     };
     // the wave's weight scales of stage s: each half-wave brings the 512 bytes of one tile (the last
     // stage's: 64 bytes per block)
@@ -765,7 +760,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void q8_rows_gemm_kernel(GemmArgs 
     if constexpr (FLAGGED) {
         int f = 0;
         if (lane < live)
-            f = *reinterpret_cast<const int *>(A.rows_in + static_cast<uint64_t>(row_off16(A, it, lane)) * 16 + A.lay.flag_offset());
+            f = *reinterpret_cast<const int *>(job_row(A, it, lane) + A.lay.flag_offset());
         flagged = __any(f != 0);
     }
 

@@ -201,16 +201,6 @@ void launch_gemv(const GemvArgs & a, hipStream_t stream);
 void launch_job_tiles(const GroupBuffers & g, const int32_t * filter, int job_tile, int64_t max_tiles,
                       int32_t * tile_expert, int32_t * tile_start, int32_t * n_tiles, hipStream_t stream);
 
-// Activation row of the MFMA grouped GEMM: row-major codes (f16 for MXFP4 weights, int8 for
-// Q8_0), fp16-rounded fp32 block scales, and the row's -128 flag; 256-byte aligned stride.
-struct GemmRowLayout {
-    int64_t nb;
-    int weight_type;
-    VBM_HD int64_t code_bytes() const { return nb * 32 * (weight_type == 39 ? 2 : 1); }
-    VBM_HD int64_t da_offset() const { return code_bytes(); }
-    VBM_HD int64_t flag_offset() const { return da_offset() + 4 * nb; }
-    VBM_HD int64_t stride() const { return (flag_offset() + 4 + 255) / 256 * 256; }
-};
 void launch_gemm_rows_from_f32(const float * x, int64_t n_rows, int64_t k, int64_t x_stride, const GemmRowLayout & lay,
                                uint8_t * rows, hipStream_t stream);
 void launch_gemm_rows_from_q8(const uint8_t * q8, int64_t n_rows, int64_t row_bytes, const GemmRowLayout & lay,
