@@ -50,3 +50,38 @@ def test_loads_to_lds_are_a_wait_state_behind_their_m0_write(device_asm):
         since = 0 if re.match(r"s_\w+ m0,", line) else since + wait_states(line)
     assert loads > 0
     assert not bad, (len(bad), bad[:3])
+
+
+def registers(operand):
+    m = re.match(r"v\[(\d+):(\d+)\]|v(\d+)\b", operand.strip())
+    if not m:
+        return set()
+    return set(range(int(m.group(1)), int(m.group(2)) + 1)) if m.group(1) else {int(m.group(3))}
+
+
+def test_matrix_results_stay_whole_until_the_inline_sum_that_reads_them(device_asm):
+    """A matrix instruction writes its registers some wait states late. The compiler keeps its own writes to
+    a result's free lanes apart from that, and inline assembly's not: a result that an inline sum reads has to
+    keep all its lanes up to the sum."""
+    pending, sums, bad, inline = [], 0, [], False
+    for line in device_asm("vbm_gemv.hip"):
+        if line.startswith(";;"):
+            inline = line.startswith(";;#ASMSTART")
+            continue
+        op, _, rest = line.partition(" ") if " " in line else line.partition("\t")
+        operands = re.split(r",(?![^\[]*\])", rest)
+        writes = registers(operands[0]) if re.match(r"v_(?!cmp)|ds_read|buffer_load|global_load|scratch_load", op) else set()
+        reads = set().union(*(registers(o) for o in operands[1:]))
+        for result in pending[:]:
+            if reads & result["regs"]:
+                if inline:
+                    sums += 1
+                    bad += [result["line"]] if result["lost"] else []
+                pending.remove(result)
+            elif writes & result["regs"]:
+                result["lost"] = True
+        if op.startswith("v_mfma_f32_4x4x4"):
+            pending.append({"line": line, "regs": writes, "lost": False})
+            del pending[:-8]
+    assert sums > 0
+    assert not bad, (len(bad), bad[:3])

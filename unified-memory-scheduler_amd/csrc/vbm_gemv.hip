@@ -393,15 +393,20 @@ __device__ __forceinline__ float row_bcast(float v) {
 // acc[m][PAR] = fma(row_bcast<N>(d[m]), v[m], acc[m][PAR]) for every token. The compiler does not fold a row
 // broadcast into an FMA (a move per token otherwise, as many as the FMAs), so the instructions are written
 // out. The s_nop ahead of them stands in for the wait states the compiler gives its own instructions: five
-// between a two-pass MFMA and a read of its result, two between a VALU write and a DPP read of it.
+// between a two-pass MFMA and a read of its result, two between a VALU write and a DPP read of it. Widths
+// below four name the MFMA's unused result lanes too: a lane that is free before those five wait states are over
+// could be given to another block's exp2_byte, which the compiler cannot hold back, and the matrix core
+// would write over it.
 #define VBM_FMAC_BCAST(acc, d, v) "v_fmac_f32_dpp %" #acc ", %" #d ", %" #v " row_newbcast:%c[n] row_mask:0xf bank_mask:0xf\n\t"
 template <int M, int PAR, int N>
 __device__ __forceinline__ void fma_bcast(float (&acc)[M][2], const float (&d)[M], const f32x4_t (&v)[(M + 3) / 4]) {
     if constexpr (M == 1)
-        asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 1, 2) : "+v"(acc[0][PAR]) : "v"(d[0]), "v"(v[0][0]), [n] "n"(N));
+        asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 1, 2)
+            : "+v"(acc[0][PAR]) : "v"(d[0]), "v"(v[0][0]), "v"(v[0][1]), "v"(v[0][2]), "v"(v[0][3]), [n] "n"(N));
     else if constexpr (M == 2)
         asm("s_nop 4\n\t" VBM_FMAC_BCAST(0, 2, 4) VBM_FMAC_BCAST(1, 3, 5)
-            : "+v"(acc[0][PAR]), "+v"(acc[1][PAR]) : "v"(d[0]), "v"(d[1]), "v"(v[0][0]), "v"(v[0][1]), [n] "n"(N));
+            : "+v"(acc[0][PAR]), "+v"(acc[1][PAR])
+            : "v"(d[0]), "v"(d[1]), "v"(v[0][0]), "v"(v[0][1]), "v"(v[0][2]), "v"(v[0][3]), [n] "n"(N));
     else {
 #pragma unroll
         for (int g = 0; g < M / 4; ++g)
