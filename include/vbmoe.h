@@ -241,7 +241,8 @@ vbm_status vbm_glu(int activation, const float * gate, const float * up, float *
 
 /* Router: logits (given, or W_r . x with W_r fp32 [n_expert][k_hidden] and optional bias,
  * computed in the ggml x86 vec_dot_f32 order) -> top-k (value desc, then lower index:
- * tools/trace/topk-tie-probe.cpp:111-113) -> softmax over the k selected
+ * tools/trace/topk-tie-probe.cpp:111-113; NaN ranks as -inf here and in every call that routes, so
+ * ids are always valid) -> softmax over the k selected
  * (gpt-oss SOFTMAX_WEIGHT gating). If `router_w` is NULL the `logits` input is used;
  * otherwise logits are written to `logits` (may be NULL). ids [n_tokens][k] int32,
  * weights [n_tokens][k] fp32. `normalize` = 0 gives plain softmax-over-selected. */

@@ -77,6 +77,40 @@ def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, exp
     layer.destroy()
 
 
+def test_nan_logits_route_alike_on_every_path(gpu):
+    """NaN logits rank as -inf: valid ids, and the same ids, weights and output from the decode kernels, the
+    batched path and a row of a batch, with as many numbers as picks, fewer, none, and real -inf among them."""
+    experts, top_k, hidden = 20, 4, 128
+    layer = Layer(gpu, H.MX, hidden, 128, experts, top_k, seed=37, router=False)
+    inf, nan = np.float32(np.inf), np.float32(np.nan)
+    logits = np.full((5, experts), nan, np.float32)
+    logits[0] = gpu.synth_normal(37, 7, 0, experts)
+    logits[0, ::3] = nan
+    logits[1, [3, 17]] = 1.0, 2.0
+    logits[3, [0, 9, 12]] = -inf, 0.5, -inf
+    logits[4, 5:] = -inf
+    x = gpu.synth_normal(37, 6, 0, 5 * hidden).reshape(5, hidden)
+    want = np.argsort(-np.where(np.isnan(logits), -inf, logits), axis=1, kind="stable")[:, :top_k]
+    batch = layer.forward_gpu(x, logits)
+    assert np.array_equal(batch[1], want)
+    d = layer.desc()
+    need = C.c_size_t()
+    gpu.call("vbm_moe_layer_workspace", C.byref(d), 1, C.byref(need))
+    work = gpu.DeviceBuffer(need.value)
+    for t in range(5):
+        dl = gpu.DeviceBuffer.from_array(logits[t:t + 1])
+        for pad in (0, 1):
+            dx = gpu.DeviceBuffer.from_array(np.concatenate([np.zeros(pad, np.float32), x[t]]))
+            out, ids, w = gpu.DeviceBuffer(4 * hidden), gpu.DeviceBuffer(4 * top_k), gpu.DeviceBuffer(4 * top_k)
+            gpu.call("vbm_moe_layer_forward", C.byref(d), dx.ptr + 4 * pad, dl.ptr, 1, out.ptr, ids.ptr, w.ptr, work.ptr, need.value, None)
+            gpu.call("vbm_stream_synchronize", None)
+            for got, ref in ((out.download(np.float32, (hidden,)), batch[0][t]), (ids.download(np.int32, (top_k,)), batch[1][t]),
+                             (w.download(np.float32, (top_k,)), batch[2][t])):
+                assert np.array_equal(got, ref, equal_nan=got.dtype == np.float32), (t, pad)
+    assert np.all(batch[2][1, 2:] == 0) and np.all(np.isnan(batch[0][2])) and not np.any(np.isnan(batch[0][[0, 1, 3]]))
+    layer.destroy()
+
+
 @pytest.mark.parametrize("top_k,hidden", [(1, 320), (8, 256), (9, 320), (17, 64)])
 def test_decode_step_finish_matches_layer_calls(gpu, top_k, hidden):
     """The step's last launch combines the ranks in batches of eight and hands out ids and weights: two

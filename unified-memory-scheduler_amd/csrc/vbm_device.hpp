@@ -23,7 +23,11 @@ __device__ __forceinline__ float glu(int activation, float g0, float u0, float a
     return g0 / (1.0f + expf_rn(-g0)) * u0;
 }
 
-// One wavefront: top-k of `logits[0..n)` in the total order (value desc, then lower index;
+// Routing logit as every top-k here reads it: NaN as -inf, so that the order is total and each pick a valid
+// index whichever kernel routes (a NaN among too few numbers is picked with weight 0).
+__device__ __forceinline__ float route_key(float v) { return v != v ? -INFINITY : v; }
+
+// One wavefront: top-k of `logits[0..n)` (route_key) in the total order (value desc, then lower index;
 // tools/trace/topk-tie-probe.cpp:111-113), pick j being the best element strictly after pick j-1,
 // then ggml soft_max over the k selected values (expf(v - max), sum in double, scale by
 // (float)(1/sum)). Lanes 0..k-1 write ids[0..k) and weights[0..k), and the ids to `ids_lds` too
@@ -40,7 +44,7 @@ __device__ __forceinline__ void wave_topk_softmax(const float * logits, int n, i
     // round.
     float lv[NPL];
 #pragma unroll
-    for (int c = 0; c < NPL; ++c) lv[c] = lane + 64 * c < n ? logits[lane + 64 * c] : 0.0f;
+    for (int c = 0; c < NPL; ++c) lv[c] = lane + 64 * c < n ? route_key(logits[lane + 64 * c]) : 0.0f;
     for (int j = 0; j < k; ++j) {
         float best = 0.0f;
         int best_i = -1;
@@ -115,9 +119,6 @@ __device__ __forceinline__ float half_wave_max(float v) {
 }
 
 constexpr int kMaxRouteExperts = 1024;
-
-// Routing logit as staged for the rank count: NaN reads as -inf so the ranks stay a permutation.
-__device__ __forceinline__ float route_key(float v) { return v != v ? -INFINITY : v; }
 
 // Whole-workgroup top-k over n <= kMaxRouteExperts logits already staged in s_val (route_key) with
 // s_rank zeroed, in the total order (value desc, then lower index;
