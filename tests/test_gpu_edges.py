@@ -47,12 +47,31 @@ def test_router_logits_bitwise(gpu, orc, n_expert, tokens, hidden):
     assert np.array_equal(di.download(np.int32, (tokens, 2)), ids)
 
 
-@pytest.mark.parametrize("type_id,hidden,inter,experts,top_k,act,biases", [
-    (H.MX, 2880, 2880, 32, 4, 1, True), (H.Q8, 2048, 768, 128, 8, 0, False), (H.MX, 64, 4096, 300, 3, 0, True),
-    (H.Q8, 4096, 64, 9, 9, 1, True), (H.MX, 448, 192, 5, 1, 1, False)])
-def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, experts, top_k, act, biases):
-    """A one-token call runs the decode kernels when its input is 16-byte aligned and the batched path
-    otherwise: the oracle's bits from both."""
+def kernels_of(gpu, call):
+    """Kernel launches that call(stream) records into a captured graph (not run)."""
+    with open("/proc/self/maps") as maps:                       # the runtime the library itself runs on
+        hip = C.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    stream, graph, count = C.c_void_p(), C.c_void_p(), C.c_size_t()
+    gpu.call("vbm_stream_create", C.byref(stream))
+    assert hip.hipStreamBeginCapture(stream, 2) == 0            # relaxed
+    call(stream.value)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    gpu.call("vbm_stream_destroy", stream.value)
+    return count.value
+
+
+@pytest.mark.parametrize("type_id,hidden,inter,experts,top_k,act,biases,decode", [
+    (H.MX, 2880, 2880, 32, 4, 1, True, True), (H.Q8, 2048, 768, 128, 8, 0, False, True), (H.MX, 64, 4096, 300, 3, 0, True, True),
+    (H.Q8, 4096, 64, 9, 9, 1, True, True), (H.MX, 448, 192, 5, 1, 1, False, True),
+    # top_k and top_k + 1 at the line between the paths, up to 128, 256 and more experts
+    (H.MX, 128, 512, 64, 32, 1, True, True), (H.MX, 128, 512, 64, 33, 1, True, False),
+    (H.Q8, 64, 512, 200, 25, 0, False, True), (H.Q8, 64, 512, 200, 26, 0, False, False),
+    (H.MX, 64, 512, 300, 16, 1, False, True), (H.MX, 64, 512, 300, 17, 1, False, False)])
+def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, experts, top_k, act, biases, decode):
+    """A one-token call runs the decode kernels (three launches) when its input is 16-byte aligned and its
+    routing small, and the batched path (four) otherwise: the oracle's bits from both, and the same ids and weights."""
     layer = Layer(gpu, type_id, hidden, inter, experts, top_k, seed=91, router=False, biases=biases, activation=act,
                   q8_scale=(1e-4, 1e-3))
     x = gpu.synth_normal(91, 6, 0, hidden).reshape(1, hidden)
@@ -66,14 +85,22 @@ def test_one_token_layer_takes_either_path(gpu, orc, type_id, hidden, inter, exp
     dx = gpu.DeviceBuffer.from_array(x)
     off = gpu.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x[0]]))
     dl = gpu.DeviceBuffer.from_array(logits)
-    for src in (dx.ptr, off.ptr + 4):
+    weights = []
+    for src, launches in ((dx.ptr, 3 if decode else 4), (off.ptr + 4, 4)):
         out, ids, w = gpu.DeviceBuffer(4 * hidden), gpu.DeviceBuffer(4 * top_k), gpu.DeviceBuffer(4 * top_k)
-        gpu.call("vbm_moe_layer_forward", C.byref(d), src, dl.ptr, 1, out.ptr, ids.ptr, w.ptr, work.ptr, need.value, None)
+
+        def forward(stream):
+            gpu.call("vbm_moe_layer_forward", C.byref(d), src, dl.ptr, 1, out.ptr, ids.ptr, w.ptr, work.ptr, need.value, stream)
+
+        assert kernels_of(gpu, forward) == launches
+        forward(None)
         gpu.call("vbm_stream_synchronize", None)
         assert np.array_equal(ids.download(np.int32, (1, top_k)), ref["ids"])
-        assert np.allclose(w.download(np.float32, (1, top_k)), ref["weights"], rtol=1e-6, atol=0)
+        weights.append(w.download(np.float32, (1, top_k)))
+        assert np.allclose(weights[-1], ref["weights"], rtol=1e-6, atol=0)
         got = out.download(np.float32, (1, hidden))
         assert H.bits_equal(got, ref["out"]), H.diff_report(got, ref["out"])
+    assert H.bits_equal(*weights)
     layer.destroy()
 
 

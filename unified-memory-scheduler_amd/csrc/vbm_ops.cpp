@@ -356,9 +356,16 @@ void record(void * const * events, int i, hipStream_t s) {
 // One token through the single-token decode kernels (bit-identical to the batched path), which route and
 // quantize in their own prologues: no routing, grouping or quantization launch before the weights start
 // to stream. hidden = inter = 2880, top-4 of 32 experts with the router's projection: 34 us a call
-// through the batched path, 22 us through this one.
+// through the batched path, 22 us through this one. Every workgroup of the two kernels picks the top_k experts
+// for itself, one after another over n_expert / 64 registers, and their number grows with top_k x intermediate: the
+// routing's work by top_k squared, against one routing per call in the batched path. Both paths where the line lies,
+// up to 128 experts: top-10 of 32, 4096 x 4096 61 and 64 us, top-12 75 and 71; top-32 of 128, hidden = inter = 512 26
+// and 39, top-64 67 and 64; top-12, 768 x 3072 31 and 33, top-16 41 and 38. Up to 256: top-24, 512 x 512 25 and
+// 35, top-12, 768 x 3072 38 and 34. 512: top-16, 512 x 512 35 and 37, top-24 54 and 49, top-64 297 and 104.
 bool single_token(const vbm_moe_layer_desc & d, const float * x, int64_t n_tokens) {
-    return n_tokens == 1 && d.hidden <= 4096 && d.intermediate <= 4096 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    const int64_t limit = d.n_expert <= 128 ? 524288 : (d.n_expert <= 256 ? 327680 : 131072);
+    return n_tokens == 1 && d.hidden <= 4096 && d.intermediate <= 4096 && d.top_k * d.top_k * d.intermediate <= limit &&
+           reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
 void single_token_forward(const vbm_moe_layer_desc & d, const float * x, const float * logits, float * out, int32_t * ids,
