@@ -33,6 +33,24 @@ def test_gemm_job_counts_around_the_tile_edges_exact(gpu, orc, type_id, rows, k)
     bank.destroy()
 
 
+def test_gemv_fold_check_sees_every_wave(gpu, orc):
+    """One exponent too large to fold, in each expert in another 1 KiB part of the tile pair's exponents (the
+    part one wave checks), at every chunk width: folded all the same, its weights overflow to infinity."""
+    rows, k, experts = 64, 4096, 8
+    rng = np.random.default_rng(8)
+    w = H.synth_weights(H.MX, 17, 3, experts, rows, k).reshape(experts, rows, k // 32, 17)
+    for e in range(experts):
+        w[e, 8 * e + int(rng.integers(8)), int(rng.integers(k // 32)), 0] = 150
+    bank = H.make_bank(H.MX, w.reshape(-1), experts, rows, k)
+    for tokens in (1, 2, 4, 7):
+        ids = np.tile(np.arange(experts, dtype=np.int32), (tokens, 1))
+        x = gpu.synth_normal(17, 4, tokens, tokens * k).reshape(tokens, 1, k)
+        got = H.mul_mat_id(bank, experts, x, gpu.TYPE_F32, 1, ids, experts)
+        ref = orc.mul_mat_id(H.MX, w.reshape(-1), k, rows, experts, 0, x, 1, ids, experts, tokens, experts, threads=8)
+        assert H.bits_equal(got, ref), (tokens, H.diff_report(got, ref))
+    bank.destroy()
+
+
 @pytest.mark.parametrize("n_expert,tokens,hidden", [(8, 3, 1000), (32, 1, 2880), (33, 250, 2880), (32, 257, 100), (64, 128, 960)])
 def test_router_logits_bitwise(gpu, orc, n_expert, tokens, hidden):
     """One token per weight row and, from 8192 (expert, token) pairs on, four: ragged token counts, rows of
