@@ -156,6 +156,25 @@ def test_nan_logits_route_alike_on_every_path(gpu):
     layer.destroy()
 
 
+@pytest.mark.parametrize("hidden,inter,top_k", [(2048, 1024, 20), (2048, 1024, 21), (1024, 512, 16), (1024, 512, 17), (704, 512, 3)])
+def test_decode_q8_ring_depths_bitwise(gpu, orc, hidden, inter, top_k):
+    """Q8_0 gate_up on both sides of the lines between its two ring depths: 1280 workgroups of the unrolled
+    kernel, 512 of the rolled one, and a row too short for the deep ring."""
+    layer = Layer(gpu, H.Q8, hidden, inter, top_k, top_k, seed=61, router=False, biases=False, activation=0, q8_scale=(1e-4, 1e-3))
+    x = gpu.synth_normal(61, 6, 0, hidden).reshape(1, hidden)
+    logits = gpu.synth_normal(61, 7, 0, top_k).reshape(1, top_k)
+    ref = layer.forward_cpu(orc, x, logits)
+    plan = C.c_void_p()
+    gpu.call("vbm_decode_plan_create", (gpu.MoeLayerDesc * 1)(layer.desc()), 1, C.byref(plan))
+    dx, dl, out = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer.from_array(logits), gpu.DeviceBuffer(4 * hidden)
+    gpu.call("vbm_decode_step", plan.value, dx.ptr, dl.ptr, out.ptr, None, None, None, None)
+    gpu.call("vbm_stream_synchronize", None)
+    got = out.download(np.float32, (1, hidden))
+    assert H.bits_equal(got, ref["out"]), H.diff_report(got, ref["out"])
+    gpu.call("vbm_decode_plan_destroy", plan.value)
+    layer.destroy()
+
+
 @pytest.mark.parametrize("top_k,hidden", [(1, 320), (8, 256), (9, 320), (17, 64)])
 def test_decode_step_finish_matches_layer_calls(gpu, top_k, hidden):
     """The step's last launch combines the ranks in batches of eight and hands out ids and weights: two

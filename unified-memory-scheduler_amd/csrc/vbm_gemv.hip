@@ -197,13 +197,9 @@ __device__ __forceinline__ void q8_group(const u32x4 & c, const u32x2 & m, int b
 
 // Weight groups a lane keeps in flight. Both MXFP4 decode kernels stream through a 5-deep ring
 // so compute overlaps the arrivals (120B-shape decode, A / B depth 6 / 12: 1511-1514 tok/s, 5 / 6:
-// 1600-1618, 5 / 5: 1627-1638, 6 / 4: 1540-1561, 7 / 6: 1522-1531); Q8_0 through an 8-deep one (three layers of
-// hidden 2048, inter 768, top-8: depth 4 50.3 us, 6 50.1, 8 49.2, 16 51.0). The batched kernel's depth
-// is set where it streams (gemv_chunk).
-template <int TYPE>
-constexpr int gate_up_depth() {
-    return TYPE == 39 ? 5 : 8;
-}
+// 1600-1618, 5 / 5: 1627-1638, 6 / 4: 1540-1561, 7 / 6: 1522-1531); Q8_0's down streams through an 8-deep one,
+// its gate_up through one of 4 or 8 by the launch's size (launch_gate_up_npl). The batched kernel's depth is
+// set where it streams (gemv_chunk).
 template <int TYPE>
 constexpr int down_depth() {
     return TYPE == 39 ? 5 : 8;
@@ -1144,9 +1140,8 @@ size_t decode_lds_bytes(int nb) {
 // STAGE (launches with a staging area, the deferred host tier): a workgroup whose pick is read
 // from the pinned host copy copies its tile into the staging area first and streams that copy.
 // A separate instantiation, so the resident-only kernels carry none of that code.
-template <int TYPE, int NPL, int NB, bool STAGE>
+template <int TYPE, int NPL, int NB, int D, bool STAGE>
 __global__ __launch_bounds__(kDownThreads) __attribute__((amdgpu_waves_per_eu(3))) void decode_gate_up_kernel(DecodeArgs A) {
-    constexpr int D = gate_up_depth<TYPE>();
     constexpr int kChunks = 2;                     // 8-element input chunks per thread (hidden <= 4096)
     __shared__ float red[8][32];
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
@@ -1769,16 +1764,25 @@ __global__ __launch_bounds__(kLinkThreads) void decode_link_kernel(LinkArgs A) {
     }
 }
 
+// Q8_0's ring depth: with 8 groups in flight the kernel holds fewer workgroups per CU than with 4 (88 against 72
+// registers unrolled: five against seven; 130 against 114 rolled: three against four), so it pays where the grid
+// is resident at once either way. Three layers, depth 4 against 8: hidden 2048, inter 1024, top-8 (512 workgroups)
+// 55.5 and 54.5 us, inter 2048, top-12 (1536) 110 and 119; rolled, hidden 1024, inter 512, top-8 (256) 44.5 and
+// 42.7 us, 1408, 2048, top-8 (1024) 75.8 and 91.6, 4096, 4096, top-4 (1024) 146 and 183; rolled rows of fewer
+// than six such groups 1 % slower with 8.
 template <int TYPE, int NPL, int NB>
 void launch_gate_up_npl(const DecodeArgs & a, dim3 grid, size_t lds, hipStream_t stream) {
+    constexpr int64_t kDeepGrid = 256 * (NB > 0 ? 5 : 2);
+    const bool deep = TYPE == 8 && static_cast<int64_t>(grid.x) * grid.y <= kDeepGrid && a.shape.nb >= 24;
     auto launch = [&](auto kernel) {
         if (lds > 65536)
             check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                           static_cast<int>(lds)), "decode gate_up LDS attribute");
         hipLaunchKernelGGL(kernel, grid, dim3(kDownThreads), lds, stream, a);
     };
-    if (a.stage) launch(&decode_gate_up_kernel<TYPE, NPL, NB, true>);
-    else launch(&decode_gate_up_kernel<TYPE, NPL, NB, false>);
+    constexpr int D = TYPE == 39 ? 5 : 4, kDeep = TYPE == 39 ? 5 : 8;
+    if (a.stage) deep ? launch(&decode_gate_up_kernel<TYPE, NPL, NB, kDeep, true>) : launch(&decode_gate_up_kernel<TYPE, NPL, NB, D, true>);
+    else deep ? launch(&decode_gate_up_kernel<TYPE, NPL, NB, kDeep, false>) : launch(&decode_gate_up_kernel<TYPE, NPL, NB, D, false>);
 }
 
 // Row lengths (blocks) with a fully unrolled weight stream: hidden = intermediate = 2880 (MXFP4,
