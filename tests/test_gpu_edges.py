@@ -51,6 +51,21 @@ def test_gemv_fold_check_sees_every_wave(gpu, orc):
     bank.destroy()
 
 
+@pytest.mark.parametrize("hidden", [32, 64, 96, 160, 256, 288, 512, 736, 31])
+@pytest.mark.parametrize("n_expert,tokens", [(8, 5), (128, 65)])
+def test_router_logits_row_ends_bitwise(gpu, orc, n_expert, tokens, hidden):
+    """Rows of 1, 2, 3, 5 and 8 steps (their own batch widths), of 9, 16 and 23 (full batches and a rest), and of
+    none, in both forms of the kernel."""
+    w = gpu.synth_normal(16, 1, 0, n_expert * hidden, 0.0, 0.02).reshape(n_expert, hidden)
+    x = gpu.synth_normal(16, 2, 0, tokens * hidden).reshape(tokens, hidden)
+    dw, dx = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x)
+    dl, di, dwt = (gpu.DeviceBuffer(4 * tokens * n) for n in (n_expert, 2, 2))
+    gpu.call("vbm_router_topk_softmax", dw.ptr, None, dx.ptr, hidden, dl.ptr, n_expert, tokens, 2, di.ptr, dwt.ptr, None)
+    logits, ids, _ = orc.router(router_w=w, x=x, n_expert=n_expert, n_tokens=tokens, top_k=2, hidden=hidden)
+    assert H.bits_equal(dl.download(np.float32, (tokens, n_expert)), logits)
+    assert np.array_equal(di.download(np.int32, (tokens, 2)), ids)
+
+
 @pytest.mark.parametrize("n_expert,tokens,hidden", [(8, 3, 1000), (32, 1, 2880), (33, 250, 2880), (32, 257, 100), (64, 128, 960)])
 def test_router_logits_bitwise(gpu, orc, n_expert, tokens, hidden):
     """One token per weight row and, from 8192 (expert, token) pairs on, four: ragged token counts, rows of
