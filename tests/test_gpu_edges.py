@@ -33,6 +33,28 @@ def test_gemm_job_counts_around_the_tile_edges_exact(gpu, orc, type_id, rows, k)
     bank.destroy()
 
 
+@pytest.mark.parametrize("type_id", [H.MX, H.Q8])
+@pytest.mark.parametrize("units", [5, 11, 13, 14, 23])
+def test_gemm_tile_splits_exact(gpu, orc, type_id, units):
+    """23 job tiles and 37 half tiles that hold jobs, over bank rows of 5 to 23 workgroups each: tiles in quarters
+    (115 items), in halves (253, and 299 with 481 parts), whole with even shares (322) and whole (529).
+    Unit scales: every fp32 sum is an exact integer."""
+    counts = [1, 0, 15, 16, 17, 33, 48, 63, 64, 65, 80, 81, 96, 97, 128, 129]
+    assert sum(-(-c // 64) for c in counts) == 23 and sum(-(-c // 32) for c in counts) == 37
+    ids = np.repeat(np.arange(len(counts)), counts).astype(np.int32)
+    rng = np.random.default_rng(units)
+    rng.shuffle(ids)
+    ids = ids.reshape(-1, 1)
+    tokens, rows, k = ids.shape[0], 256 * units - 160, 192
+    w = (unit_scale_mxfp4 if type_id == H.MX else unit_scale_q8)(len(counts), rows, k, rng)
+    bank = H.make_bank(type_id, w, len(counts), rows, k)
+    x = unit_scale_activations(tokens, k, rng).reshape(tokens, 1, k)
+    got = H.mul_mat_id(bank, len(counts), x, gpu.TYPE_F32, 1, ids, 1, order=gpu.ORDER_FAST)
+    ref = orc.mul_mat_id(type_id, w, k, rows, len(counts), 0, x, 1, ids, 1, tokens, 1, threads=8)
+    assert H.bits_equal(got, ref), H.diff_report(got, ref)
+    bank.destroy()
+
+
 def test_gemv_fold_check_sees_every_wave(gpu, orc):
     """One exponent too large to fold, in each expert in another 1 KiB part of the tile pair's exponents (the
     part one wave checks), at every chunk width: folded all the same, its weights overflow to infinity."""

@@ -24,6 +24,7 @@
 // int-to-float conversions (Q8_0) come on top, so the layout keeps everything else off it: weights
 // in registers (no address or LDS work per operand), 64-row waves (four MFMAs per activation read) and
 // sums placed under the MFMAs.
+#include <algorithm>
 #include <type_traits>
 
 #include "vbm_device.hpp"
@@ -230,25 +231,56 @@ struct RowsItem {
     int expert, j0, joff, live, slot, pair0;
 };
 
-// XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of (tile, row unit)
-// items; the units of one job tile share its activation rows in one L2. False: no item, or one whose
-// expert is not resident in this bank. The latter writes NaN outputs, as the decode kernels do (a tile
-// filter removes the experts a pass skips on purpose, so this is a bad map).
+// Workgroups that the card holds at once (two per CU by LDS). A launch that leaves places free splits every job
+// tile into halves or quarters of 32 or 16 jobs, as long as the parts that hold jobs fit: a workgroup's K loop is
+// then as long as its one or two fragment columns, not four, on CUs that would otherwise be idle or hold one of
+// the few second workgroups. The parts read the same weights, from L2. One expert of 4096 x 4096 and 64 tokens (16
+// items): Q8_0 66.8 -> 35 us, MXFP4 60.5 -> 38; 1024 tokens over 16 experts of 2880 x 2880 (288): Q8_0 79 -> 73 us.
+constexpr int kGemmSlots = 512;
+
+// log2 of the parts of each job tile for n_tiles tiles. Called by whole waves.
+__device__ __forceinline__ int tile_split(const GemmArgs & A, int job_tile, int n_tiles) {
+    const int whole = n_tiles * A.row_units;
+    if (whole * 4 <= kGemmSlots) return 2;
+    if (whole * 2 <= kGemmSlots) return 1;
+    if (whole > kGemmSlots) return 0;
+    int parts = 0;                                           // halves that hold jobs
+    for (int i = threadIdx.x & 63; i < n_tiles; i += 64)
+        parts += A.counts[A.tile_expert[i]] - A.tile_start[i] > job_tile / 2 ? 2 : 1;
+    for (int off = 32; off > 0; off >>= 1) parts += __shfl_xor(parts, off);
+    return __builtin_amdgcn_readfirstlane(parts) * A.row_units <= kGemmSlots ? 1 : 0;
+}
+
+// XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of (tile, row unit, part)
+// items; the units of one job tile share its activation rows in one L2, its parts their weights. False: no item,
+// or one whose expert is not resident in this bank. The latter writes NaN outputs, as the decode kernels do (a
+// tile filter removes the experts a pass skips on purpose, so this is a bad map).
 template <int EPI>
 __device__ __forceinline__ bool rows_item(const GemmArgs & A, int job_tile, RowsItem & it) {
-    const int n_items = *cst<int32_t>(A.n_tiles) * A.row_units;
+    const int n_tiles = *cst<int32_t>(A.n_tiles), split = tile_split(A, job_tile, n_tiles);
+    const int n_items = n_tiles * A.row_units << split;
     const int per_xcd = (n_items + 7) >> 3;
     const int slot8 = static_cast<int>(blockIdx.x >> 3);
-    const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
-    if (slot8 >= per_xcd || item >= n_items) return false;
-    const int ti = item / A.row_units;
+    const int part = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
+    if (slot8 >= per_xcd || part >= n_items) return false;
+    const int item = part >> split, ti = item / A.row_units;
     it.pair0 = (item - ti * A.row_units) * 4;
     it.expert = cst<int32_t>(A.tile_expert)[ti];
-    it.j0 = cst<int32_t>(A.tile_start)[ti];
     const int count = cst<int32_t>(A.counts)[it.expert];
+    int t0 = cst<int32_t>(A.tile_start)[ti], share = job_tile;
+    if (n_items <= kGemmSlots) {
+        // all items run at once: an expert's tiles share its jobs evenly, in fragment columns of 16, so that
+        // 80 jobs run as 48 + 32, not 64 + 16 (80 jobs each of 24 experts, 1536 x 4096: Q8_0 107 -> 92 us)
+        const int tiles = (count + job_tile - 1) / job_tile;
+        share = ((count + tiles - 1) / tiles + 15) & ~15;
+        t0 = t0 / job_tile * share;
+    }
+    const int p0 = (part - (item << split)) * (job_tile >> split);
+    it.j0 = t0 + p0;
     it.joff = cst<int32_t>(A.offsets)[it.expert];
     it.slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[it.expert] : it.expert;
-    it.live = count - it.j0 < job_tile ? count - it.j0 : job_tile;
+    it.live = std::min(std::min(count - t0, share) - p0, job_tile >> split);
+    if (it.live <= 0) return false;                          // a part past the tile's last job
     const GemmShape & S = A.shape;
     if (it.slot >= 0 && it.slot < S.n_slots) return true;
     const float nan = __builtin_nanf("");
@@ -1076,7 +1108,9 @@ template <int TYPE, int EPI, bool FLAGGED>
 void launch_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
     GemmArgs b = a;
     b.row_units = static_cast<int>((rows + 255) / 256);
-    const int64_t items = static_cast<int64_t>(b.row_units) * max_tiles;
+    // whole tiles, or their parts where the actual tiles are few (rows_item)
+    const int64_t whole = static_cast<int64_t>(b.row_units) * max_tiles;
+    const int64_t items = std::max(whole, std::min<int64_t>(whole * 4, 2 * kGemmSlots));
     const dim3 grid(static_cast<unsigned>((items + 7) / 8 * 8));
     if constexpr (TYPE == 39) hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
     else hipLaunchKernelGGL((q8_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
