@@ -302,8 +302,10 @@ vbm_status vbm_moe_layer_forward(const vbm_moe_layer_desc * desc, const float * 
                                  size_t workspace_bytes, void * stream);
 
 /* Same as vbm_moe_layer_forward, also recording events[0..3] (hipEvent_t as void*) on `stream`
- * immediately before/after the gate_up GEMV and before/after the down GEMV, so callers can time
- * the two dominant kernels over a live run. No reference counterpart (profiling hook, the
+ * immediately before/after the gate_up kernel and before/after the down kernel, so callers can time
+ * the two dominant kernels over a live run. A one-token call may run the decode kernels (A and B
+ * below): its first pair then brackets the routing and the input quantization too, which that
+ * kernel does itself, and the second pair the quantization of the GLU outputs. No reference counterpart (profiling hook, the
  * analogue of the scheduler counters of hybrid-experts.patch:143-172). */
 vbm_status vbm_moe_layer_forward_profiled(const vbm_moe_layer_desc * desc, const float * x,
                                           float * logits, int64_t n_tokens, float * out,
