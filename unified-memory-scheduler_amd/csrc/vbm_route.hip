@@ -335,6 +335,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float * __rest
 #pragma unroll
             for (int t = 0; t < TT; ++t) xv[t][u] = xr[t][i];
         }
+        __builtin_amdgcn_sched_barrier(0);                   // (left to itself the compiler sums as it loads)
 #pragma unroll
         for (int u = 0; u < N; ++u)
             if (i0 + 32 * u < np) {
