@@ -1765,15 +1765,16 @@ __global__ __launch_bounds__(kLinkThreads) void decode_link_kernel(LinkArgs A) {
 }
 
 // Q8_0's ring depth: with 8 groups in flight the kernel holds fewer workgroups per CU than with 4 (88 against 72
-// registers unrolled: five against seven; 130 against 114 rolled: three against four), so it pays where the grid
-// is resident at once either way. Three layers, depth 4 against 8: hidden 2048, inter 1024, top-8 (512 workgroups)
+// registers unrolled: five against seven; 130 against 114 rolled: three against four), so it takes the grids that
+// run in as many rounds either way. Three layers, depth 4 against 8: hidden 2048, inter 1024, top-8 (512 workgroups)
 // 55.5 and 54.5 us, inter 2048, top-12 (1536) 110 and 119; rolled, hidden 1024, inter 512, top-8 (256) 44.5 and
-// 42.7 us, 1408, 2048, top-8 (1024) 75.8 and 91.6, 4096, 4096, top-4 (1024) 146 and 183; rolled rows of fewer
-// than six such groups 1 % slower with 8.
+// 42.7 us, 1408, 2048, top-8 (1024) 75.8 and 91.6, top-12 (1536) 115.8 and 113.5, 4096, 4096, top-4 (1024) 146 and 183.
+// Rolled rows of fewer than six such groups are 1 % slower with 8.
 template <int TYPE, int NPL, int NB>
 void launch_gate_up_npl(const DecodeArgs & a, dim3 grid, size_t lds, hipStream_t stream) {
-    constexpr int64_t kDeepGrid = 256 * (NB > 0 ? 5 : 2);
-    const bool deep = TYPE == 8 && static_cast<int64_t>(grid.x) * grid.y <= kDeepGrid && a.shape.nb >= 24;
+    const int64_t wgs = static_cast<int64_t>(grid.x) * grid.y;
+    auto rounds = [&](int per_cu) { return (wgs + 256 * per_cu - 1) / (256 * per_cu); };
+    const bool deep = TYPE == 8 && a.shape.nb >= 24 && (NB > 0 ? rounds(5) == rounds(7) : rounds(3) == rounds(4));
     auto launch = [&](auto kernel) {
         if (lds > 65536)
             check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
