@@ -228,7 +228,7 @@ struct GemmRowLayout {
     VBM_HD int64_t flag_offset() const { return da_offset() + 4 * nb; }
     VBM_HD int64_t stride() const { return (flag_offset() + 4 + 255) / 256 * 256; }
     // Byte offset of a row: the rows that a launch admits go past 64 GiB.
-    VBM_HD uint64_t row_offset(uint32_t row) const { return static_cast<uint64_t>(row) * static_cast<uint64_t>(stride()); }
+    VBM_HD uint64_t row_offset(uint32_t row) const { return static_cast<uint64_t>(row) * static_cast<uint32_t>(stride()); }
 };
 
 }  // namespace vbm

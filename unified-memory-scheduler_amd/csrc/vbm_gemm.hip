@@ -86,8 +86,8 @@ struct GemmArgs {
     const float * bias;        // [n_expert][rows] in ggml row order, or null
     const float * row_scale;   // epilogue 0: per-job factor applied after the bias (routing weights), or null
     float * dst;               // epilogue 0: [job][rows]
-    int row_pairs;             // 64-row tile pairs of the bank
-    int row_units;             // MXFP4: 256-row units of the bank
+    int row_units;             // 256-row units of the bank
+    int split;                 // log2 of the most parts a job tile may run in (rows_item)
     uint8_t * rows_out;        // epilogue 1: GLU output rows for the down projection (out_lay)
     GemmRowLayout out_lay;
     int activation;
@@ -231,51 +231,47 @@ struct RowsItem {
     int expert, j0, joff, live, slot, pair0;
 };
 
-// Workgroups that the card holds at once (two per CU by LDS). A launch that leaves places free splits every job
-// tile into halves or quarters of 32 or 16 jobs, as long as the parts that hold jobs fit: a workgroup's K loop is
-// then as long as its one or two fragment columns, not four, on CUs that would otherwise be idle or hold one of
-// the few second workgroups. The parts read the same weights, from L2. One expert of 4096 x 4096 and 64 tokens (16
-// items): Q8_0 66.8 -> 35 us, MXFP4 60.5 -> 38; 1024 tokens over 16 experts of 2880 x 2880 (288): Q8_0 79 -> 73 us.
+// Workgroups that the card holds at once (two per CU by LDS). A launch of few items splits every job tile into
+// quarters or halves of 16 or 32 jobs (at most as the launch allows): a workgroup's K loop
+// is then as long as its one or two fragment columns, not four, on CUs that would otherwise be idle, and the parts
+// read the same weights, from L2. One expert of 4096 x 4096 and 64 tokens (16 items): Q8_0 66.8 -> 35 us, MXFP4 60.5 ->
+// 38; 128 items, 32 jobs an expert: 59 -> 51 and 54 -> 49. Halves pay while CUs are left over: 64 rows for each of 8
+// experts of 2880 x 2880 (142 items) Q8_0 57 -> 51 us; with one workgroup per CU already (256 items, 48 jobs) they
+// took 93 against 78.
 constexpr int kGemmSlots = 512;
-
-// log2 of the parts of each job tile for n_tiles tiles. Called by whole waves.
-__device__ __forceinline__ int tile_split(const GemmArgs & A, int job_tile, int n_tiles) {
-    const int whole = n_tiles * A.row_units;
-    if (whole * 4 <= kGemmSlots) return 2;
-    if (whole * 2 <= kGemmSlots) return 1;
-    if (whole > kGemmSlots) return 0;
-    int parts = 0;                                           // halves that hold jobs
-    for (int i = threadIdx.x & 63; i < n_tiles; i += 64)
-        parts += A.counts[A.tile_expert[i]] - A.tile_start[i] > job_tile / 2 ? 2 : 1;
-    for (int off = 32; off > 0; off >>= 1) parts += __shfl_xor(parts, off);
-    return __builtin_amdgcn_readfirstlane(parts) * A.row_units <= kGemmSlots ? 1 : 0;
+__host__ __device__ __forceinline__ int tile_split(int n_items, int most) {   // log2 of a tile's parts
+    const int fits = n_items * 4 <= kGemmSlots ? 2 : (n_items * 2 <= kGemmSlots - kGemmSlots / 8 ? 1 : 0);
+    return fits < most ? fits : most;
 }
 
-// XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of (tile, row unit, part)
-// items; the units of one job tile share its activation rows in one L2, its parts their weights. False: no item,
-// or one whose expert is not resident in this bank. The latter writes NaN outputs, as the decode kernels do (a
-// tile filter removes the experts a pass skips on purpose, so this is a bad map).
+// XCD-aware order: workgroup i runs on XCD i % 8, so each XCD takes a contiguous range of (tile, row unit) items;
+// the units of one job tile share its activation rows in one L2. An XCD's first parts come before its second ones:
+// the parts without jobs are then the last, not every other one, which left the live ones on every other CU (85
+// tokens top-4 over 15 experts of 2880 x 2880: 110 against 80 us). False: no item, or one whose expert is not
+// resident in this bank. The latter writes NaN outputs, as the decode kernels do (a tile filter removes the experts a
+// pass skips on purpose, so this is a bad map).
 template <int EPI>
 __device__ __forceinline__ bool rows_item(const GemmArgs & A, int job_tile, RowsItem & it) {
-    const int n_tiles = *cst<int32_t>(A.n_tiles), split = tile_split(A, job_tile, n_tiles);
-    const int n_items = n_tiles * A.row_units << split;
+    const int n_items = *cst<int32_t>(A.n_tiles) * A.row_units, split = tile_split(n_items, A.split);
     const int per_xcd = (n_items + 7) >> 3;
     const int slot8 = static_cast<int>(blockIdx.x >> 3);
-    const int part = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8;
-    if (slot8 >= per_xcd || part >= n_items) return false;
-    const int item = part >> split, ti = item / A.row_units;
+    if (slot8 >= per_xcd << split) return false;
+    const int part = slot8 >= 2 * per_xcd ? (slot8 >= 3 * per_xcd ? 3 : 2) : (slot8 >= per_xcd ? 1 : 0);
+    const int item = static_cast<int>(blockIdx.x & 7) * per_xcd + slot8 - part * per_xcd;
+    if (item >= n_items) return false;
+    const int ti = item / A.row_units;
     it.pair0 = (item - ti * A.row_units) * 4;
     it.expert = cst<int32_t>(A.tile_expert)[ti];
     const int count = cst<int32_t>(A.counts)[it.expert];
     int t0 = cst<int32_t>(A.tile_start)[ti], share = job_tile;
-    if (n_items <= kGemmSlots) {
+    if (count > job_tile && n_items <= kGemmSlots) {
         // all items run at once: an expert's tiles share its jobs evenly, in fragment columns of 16, so that
         // 80 jobs run as 48 + 32, not 64 + 16 (80 jobs each of 24 experts, 1536 x 4096: Q8_0 107 -> 92 us)
         const int tiles = (count + job_tile - 1) / job_tile;
         share = ((count + tiles - 1) / tiles + 15) & ~15;
         t0 = t0 / job_tile * share;
     }
-    const int p0 = (part - (item << split)) * (job_tile >> split);
+    const int p0 = part * (job_tile >> split);
     it.j0 = t0 + p0;
     it.joff = cst<int32_t>(A.offsets)[it.expert];
     it.slot = A.expert_to_slot ? cst<int32_t>(A.expert_to_slot)[it.expert] : it.expert;
@@ -1104,14 +1100,19 @@ __global__ __launch_bounds__(256) void gemm_rows_from_q8_kernel(const uint8_t * 
     if (threadIdx.x == 0) *reinterpret_cast<int *>(o + L.flag_offset()) = s_flag;
 }
 
+// `experts` with jobs at most, `entries` jobs in all. Parts of 16 or 32 jobs are launched where the experts hold
+// more on average and the tiles are likely few enough (a grid of 512 for 140 workgroups with jobs cost a layer's two
+// launches 2 us of 50).
 template <int TYPE, int EPI, bool FLAGGED>
-void launch_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, hipStream_t stream) {
+void launch_rows_gemm(const GemmArgs & a, int64_t rows, int max_tiles, int64_t experts, int64_t entries, hipStream_t stream) {
     GemmArgs b = a;
     b.row_units = static_cast<int>((rows + 255) / 256);
-    // whole tiles, or their parts where the actual tiles are few (rows_item)
-    const int64_t whole = static_cast<int64_t>(b.row_units) * max_tiles;
-    const int64_t items = std::max(whole, std::min<int64_t>(whole * 4, 2 * kGemmSlots));
-    const dim3 grid(static_cast<unsigned>((items + 7) / 8 * 8));
+    const int64_t mean = entries / experts, whole = static_cast<int64_t>(b.row_units) * max_tiles;
+    const int64_t likely = std::min(whole, b.row_units * experts * ((mean + 63) / 64));
+    b.split = mean > 16 && likely * 4 <= kGemmSlots ? 2 : (mean > 32 && likely * 2 <= kGemmSlots ? 1 : 0);
+    // every tile that there can be, or the parts of so few of them that they are split
+    const int64_t tiles = (whole + 7) / 8 * 8;
+    const dim3 grid(static_cast<unsigned>(std::max(tiles, std::min<int64_t>(tiles << b.split, b.split ? kGemmSlots : 0))));
     if constexpr (TYPE == 39) hipLaunchKernelGGL((mx_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
     else hipLaunchKernelGGL((q8_rows_gemm_kernel<EPI, FLAGGED>), grid, dim3(kGemmThreads), 0, stream, b);
     check_hip(hipGetLastError(), "grouped GEMM launch");
@@ -1485,13 +1486,13 @@ void launch_grouped_gemm(const GemmParams & p, hipStream_t stream) {
     require(p.grid_tiles >= 0 && (p.grid_tiles == 0 || p.tile_filter != nullptr), "grid tile bound needs a tile filter");
     const int mt = static_cast<int>(p.grid_tiles > 0 ? std::min<int64_t>(p.grid_tiles, max_tiles) : max_tiles);
     if (bank.type == VBM_TYPE_MXFP4) {
-        if (p.flagged_rows) launch_rows_gemm<39, 0, true>(a, bank.rows, mt, stream);
-        else if (p.epilogue == 0) launch_rows_gemm<39, 0, false>(a, bank.rows, mt, stream);
-        else launch_rows_gemm<39, 1, false>(a, bank.rows, mt, stream);
+        if (p.flagged_rows) launch_rows_gemm<39, 0, true>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
+        else if (p.epilogue == 0) launch_rows_gemm<39, 0, false>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
+        else launch_rows_gemm<39, 1, false>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
     } else {
-        if (p.flagged_rows) launch_rows_gemm<8, 0, true>(a, bank.rows, mt, stream);
-        else if (p.epilogue == 0) launch_rows_gemm<8, 0, false>(a, bank.rows, mt, stream);
-        else launch_rows_gemm<8, 1, false>(a, bank.rows, mt, stream);
+        if (p.flagged_rows) launch_rows_gemm<8, 0, true>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
+        else if (p.epilogue == 0) launch_rows_gemm<8, 0, false>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
+        else launch_rows_gemm<8, 1, false>(a, bank.rows, mt, std::min(p.n_as, p.n_entries), p.n_entries, stream);
     }
 }
 
