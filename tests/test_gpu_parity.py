@@ -370,7 +370,7 @@ def test_mul_mat_id_every_chunk_width_bitwise(gpu, orc, type_id):
 
 
 def test_mul_mat_id_mxfp4_matrix_path_exponent_ranges_bitwise(gpu, orc):
-    """The MXFP4 batched GEMV runs chunks of 3..8 tokens on the matrix cores and folds the block
+    """The MXFP4 batched GEMV runs its chunks on the matrix cores and folds the block
     exponents into the weight conversion only when every exponent of a tile pair's rows lies in
     [-14, 12] (ggml e8m0 bytes 114..140); other tile pairs take ldexp per output. Per expert:
     all in range (the generator's), both boundaries (114 and 140) in range, one byte just outside

@@ -98,11 +98,10 @@ def test_gemm_power_of_two_scales_exact(gpu, orc, type_id):
 @pytest.mark.parametrize("experts,n_ids,tokens", [(2, 2, 190), (3, 2, 257), (4, 2, 300), (2, 2, 300), (2, 2, 192),
                                                    (2, 2, 193), (2, 2, 385)])
 def test_gemm_multi_tile_experts_exact(gpu, orc, type_id, experts, n_ids, tokens):
-    """Experts with 150..385 routed jobs run the grouped GEMM over one to three job tiles (128 jobs
-    for MXFP4, 192 for Q8_0: full ones and a partial last one, down to a single job), each tile's
-    live jobs split between its two wave halves. With unit scales every fp32 sum is an exact
-    integer, so the GEMM must match the oracle bit for bit, for fp32 inputs and for ggml Q8_0
-    inputs carrying -128 codes (the flagged kernel)."""
+    """Experts with 150..385 routed jobs run the grouped GEMM over three to seven job tiles of up to 64
+    jobs (full ones and a partial last one, down to a single job). With unit scales every fp32 sum is
+    an exact integer, so the GEMM must match the oracle bit for bit, for fp32 inputs and for ggml
+    Q8_0 inputs carrying -128 codes (the flagged kernel)."""
     rng = np.random.default_rng(7000 + experts)
     rows, k = 128, 256
     w = (unit_scale_mxfp4 if type_id == H.MX else unit_scale_q8)(experts, rows, k, rng)
@@ -128,7 +127,7 @@ def test_gemm_multi_tile_experts_exact(gpu, orc, type_id, experts, n_ids, tokens
 @pytest.mark.parametrize("type_id", [H.MX, H.Q8])
 def test_gemm_unaligned_destination_exact(gpu, orc, type_id):
     """A destination 4 bytes past a 16-byte boundary takes the per-element stores of the fp32
-    epilogue (aligned ones leave through the LDS tile as 16-byte stores), and fp32 activations 4
+    epilogue (aligned ones take 16-byte stores), and fp32 activations 4
     bytes past one take the scalar loads of the row quantizer: bit-identical to the oracle with
     unit scales, biases included, over a bank whose last tile pair is half live."""
     rng = np.random.default_rng(7100 + type_id)
@@ -149,7 +148,7 @@ def test_gemm_unaligned_destination_exact(gpu, orc, type_id):
 @pytest.mark.parametrize("type_id", [H.MX, H.Q8])
 def test_prefill_layer_multi_tile_experts(gpu, orc, type_id):
     """The fused layer (gate_up GEMM with the GLU + requantization epilogue, then the down GEMM)
-    with 4 experts top-2 at T = 300, so every expert holds 110..190 jobs over 2..3 job tiles:
+    with 4 experts top-2 at T = 300, so every expert holds 110..190 jobs over 2..3 job tiles of 64:
     ids exact, output within the fast order's tolerance of the oracle."""
     layer = Layer(gpu, type_id, 256, 256, 4, 2, seed=4400 + type_id, router=False,
                   activation=1 if type_id == H.MX else 0, order=gpu.ORDER_FAST)
@@ -187,6 +186,32 @@ def test_gemm_mxfp4_exponent_ranges_exact(gpu, orc):
     got = H.mul_mat_id(bank, experts, x, gpu.TYPE_F32, 1, ids, n_ids, order=gpu.ORDER_FAST)
     ref = orc.mul_mat_id(H.MX, w, k, rows, experts, 0, x, 1, ids, n_ids, tokens, n_ids, threads=8)
     assert H.bits_equal(got, ref), H.diff_report(got, ref)
+    bank.destroy()
+
+
+@pytest.mark.parametrize("k", [576, 384, 448])
+def test_gemm_mxfp4_tail_exponents_exact(gpu, orc, k):
+    """Tails of 2, 4 and 6 blocks whose exponents differ by row and block, in row tiles that fold (bytes 126..128
+    at the tail, 127 before) and that do not (140..142, and 112..114), for fp32 inputs and for ggml Q8_0 inputs
+    carrying -128 codes. A row's block scales lie within a factor of 4, so that every fp32 sum is exact."""
+    rng = np.random.default_rng(k)
+    experts, rows, n_ids, tokens = 4, 320, 2, 48
+    nb, tail = k // 32, k // 32 % 8
+    blk = unit_scale_mxfp4(experts, rows, k, rng).reshape(experts, rows, nb, 17)
+    base = np.array([127, 141, 127, 113, 127], np.uint8)[np.arange(rows) // 64]
+    blk[..., 0] = base[None, :, None]
+    blk[:, :, nb - tail:, 0] += ((np.arange(rows)[:, None] * 5 + np.arange(tail)[None, :] * 2) % 3).astype(np.uint8) - np.uint8(1)
+    bank = H.make_bank(H.MX, blk.reshape(-1), experts, rows, k)
+    ids = np.stack([rng.choice(experts, n_ids, replace=False) for _ in range(tokens)]).astype(np.int32)
+    x = unit_scale_activations(tokens, k, rng).reshape(tokens, 1, k)
+    q = orc.quantize_q8_0(x.reshape(tokens, k)).reshape(tokens, 1, -1)
+    qb = q.reshape(-1, 34)
+    qb[::3, 2 + 5] = 128
+    qb[::7, 2:10] = 128
+    for b, b_type, orc_type in ((x, gpu.TYPE_F32, 0), (q, gpu.TYPE_Q8_0, 8)):
+        got = H.mul_mat_id(bank, experts, b, b_type, 1, ids, n_ids, order=gpu.ORDER_FAST)
+        ref = orc.mul_mat_id(H.MX, blk.reshape(-1), k, rows, experts, orc_type, b, 1, ids, n_ids, tokens, n_ids, threads=8)
+        assert H.bits_equal(got, ref), (orc_type, H.diff_report(got, ref))
     bank.destroy()
 
 
@@ -308,9 +333,8 @@ def test_prefill_layer_mxfp4_config1_shape(gpu, orc):
 
 @pytest.mark.parametrize("experts,tokens", [(128, 32), (32, 24), (32, 64)])
 def test_fast_order_small_groups_take_the_exact_gemv(gpu, orc, experts, tokens):
-    """Below 12 routed rows per expert on average a fast-order call runs the exact-order GEMV
-    (faster there than the grouped GEMM): the layer output is bit-identical to the exact order's
-    and to the oracle's."""
+    """Below 12 routed rows per expert on average a fast-order call runs the exact-order GEMV: the
+    layer output is bit-identical to the exact order's and to the oracle's."""
     assert tokens * 4 < 12 * experts and tokens >= 16
     fast = Layer(gpu, H.MX, 2880, 2880, experts, 4, seed=91, router=False, order=gpu.ORDER_FAST)
     x = gpu.synth_normal(91, 6, 0, tokens * 2880).reshape(tokens, 2880)
