@@ -89,7 +89,7 @@ __device__ __forceinline__ float dpp_move(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
-// 2^(b - 127) for byte N of `w`, b its value: the byte in the f32 exponent field, one instruction by byte
+// 2^(b - 127) for byte N of `w`, b its value (0 for b = 0): the byte in the f32 exponent field, one instruction by byte
 // select (the compiler takes a shift and a mask for bytes 0..2).
 template <int N>
 __device__ __forceinline__ float exp2_byte(unsigned w) {

@@ -42,12 +42,6 @@ typedef unsigned u32x2g __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_g __attribute__((ext_vector_type(4)));
 
 constexpr int kGemmThreads = 256;
-// Jobs per grouped-GEMM workgroup (gemm_job_tile) and 16-job fragment columns per wave: the two
-// wave halves of a workgroup split its live jobs evenly.
-template <int TYPE>
-constexpr int job_tile() {
-    return TYPE == 39 ? 128 : 192;
-}
 constexpr int kMxJobTile = 64;                             // the MXFP8 experiment's job tile
 
 template <class T>
@@ -158,15 +152,6 @@ __device__ __forceinline__ half8_t i8_to_f16(long v) {
 __device__ __forceinline__ void lds_dma_x4(const void * src, uint32_t m0) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
 }
-__device__ __forceinline__ void lds_dma_x1(const void * src, uint32_t m0) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
-}
-__device__ __forceinline__ void lds_dma_x1_s(const void * base, uint32_t off, uint32_t m0) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
-}
-__device__ __forceinline__ void lds_dma_x4_s(const void * base, uint32_t off, uint32_t m0) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
-}
 #pragma clang diagnostic pop
 template <int N>
 __device__ __forceinline__ void lds_dma_wait() {
@@ -196,9 +181,11 @@ __device__ __forceinline__ float glu_fast(int activation, float g0, float u0, fl
 // one wait and one barrier per group. A workgroup takes 256 rows x one job tile.
 // Each wave's block products are summed with one FMA per output and block in block order: the split
 // over waves changes no bit of the result. One layer of 2048 tokens top-4 over 128 experts, hidden = inter =
-// 2880: gate_up 976 -> 490 us, down 502 -> 270 us against 32 x 32 waves with dword-staged weights (277 and
-// 251 TFLOP/s of block dots, from 139 and 135); two-wave workgroups of 128 rows, a stage of half a group
+// 2880: gate_up 976 -> 470..530 us, down 502 -> 255..290 us by box (512 to 578 and 468 to 533 TFLOP/s, from 278 and
+// 271) against 32 x 32 waves with dword-staged weights; two-wave workgroups of 128 rows, a stage of half a group
 // or 128-job tiles split over wave pairs measured 7 to 9 % slower.
+// Registers are full (two workgroups per CU leave 256): 31 or 32 values are spilled, around the K loop, but for
+// the kernel for caller-quantized rows, which holds both paths' code and reads four back in each group of four columns.
 //
 // The block exponents ride in the A operand when every exponent e of the wave's rows lies in
 // [-14, 12] (2^(e+1) times the e2m1 values is then an exact normal f16), which the wave checks
@@ -694,7 +681,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void mx_rows_gemm_kernel(GemmArgs 
 // four K = 4 blocks each hold one quantization block's scales at k = 0 and zeros: exact fp32 products of
 // two fp16 values, a quarter of a matrix instruction per block and nothing on the vector ALU, which is
 // left the int-to-float conversion and the FMA of every output and block. One layer of 2048 tokens top-8 over 128
-// experts, hidden 2048, inter 768: gate_up 260 -> 198 us, down 180 -> 123 us against the former 32-row waves.
+// experts, hidden 2048, inter 768: gate_up 260 -> 200..212 us, down 180 -> 122..133 us by box against the former 32-row
+// waves. 14 to 16 values are spilled, around the K loop. The kernel for caller-quantized rows spills 172: it reads ten back
+// per block of the -128 path, and in its full stages one for four columns and five for two; rows without such codes take
+// 45 to 51 us where the former kernel, which spilled none, took 94 (517 tokens x 6 ids over 64 experts, 2048 x 1408).
 struct Q8StageLayout {
     static constexpr int kJobs = 64;
     static constexpr int ROW = 8 * 32;                         // int8 codes of a job and stage
@@ -1443,9 +1433,10 @@ void launch_grouped_gemm(const GemmParams & p, hipStream_t stream) {
             "GLU epilogue needs an interleaved gate|up bank with rows % 64 == 0 and a matching output layout");
     require(p.epilogue == 1 || p.dst != nullptr, "missing GEMM output");
     require(p.n_as >= 1 && p.n_as <= 1024 && p.n_entries >= 1, "GEMM group shape out of range");
-    const int job_tile_n = gemm_job_tile(bank.type);
+    const int job_tile_n = kGemmJobTile;
     const int64_t max_tiles = gemm_max_tiles(p.n_as, p.n_entries, job_tile_n);
-    // the bound holds for tiles of 128 (MXFP4) and 192 (Q8_0) jobs, whatever tile the kernel takes
+    // calls of up to some 8.4 (MXFP4) or 12.6 (Q8_0) million entries: the limit on tiles of 128 and 192 jobs that the
+    // entry points have always had, beyond which nothing was measured
     require(gemm_max_tiles(p.n_as, p.n_entries, bank.type == VBM_TYPE_MXFP4 ? 128 : 192) <= 65535, "too many GEMM tiles for one launch");
     int32_t * tile_expert = static_cast<int32_t *>(p.tiles);
     int32_t * tile_start = tile_expert + max_tiles;

@@ -435,9 +435,8 @@ struct ActBlocks {
     }
 };
 
-// Block N of the 16 in `act`. MXFP4: bytes SEL, SEL + 1 of `w` are the slice's nibbles, `raw` its e8m0
-// exponent byte + 1 in the low byte of a word shifted into the f32 exponent field by the caller (FOLD) or the
-// signed exponent; Q8_0: `w` the four codes, dw the block's scale.
+// Block N of the 16 in `act`. MXFP4: bytes SEL, SEL + 1 of `w` are the slice's nibbles, its exponent e comes as
+// fold_scale = 2^(e + 1) (FOLD) or as it is; Q8_0: `w` the four codes, dw the block's scale.
 template <int M, int SEL, int PAR, int N, bool FOLD>
 __device__ __forceinline__ void mx_block_mm(unsigned w, float fold_scale, int e, const ActBlocks<39, M> & act, float (&acc)[M][2]) {
     const float sc = FOLD ? fold_scale : 2.0f;

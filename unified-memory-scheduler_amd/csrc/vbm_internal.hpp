@@ -232,7 +232,7 @@ struct GemmParams {
     bool tiles_ready;                 // `tiles` already holds this group's list (same group and filter)
 };
 // Jobs per grouped-GEMM workgroup (one expert's job tile): a wave's four 16-job fragment columns.
-inline int gemm_job_tile(int) { return 64; }
+constexpr int kGemmJobTile = 64;
 int64_t gemm_max_tiles(int64_t n_as, int64_t n_entries, int job_tile);
 size_t gemm_tiles_bytes(int64_t n_as, int64_t n_entries);
 void launch_grouped_gemm(const GemmParams & p, hipStream_t stream);
