@@ -226,7 +226,7 @@ struct RowsItem {
 // experts of 2880 x 2880 (142 items) Q8_0 57 -> 51 us; with one workgroup per CU already (256 items, 48 jobs) they
 // took 93 against 78.
 constexpr int kGemmSlots = 512;
-__host__ __device__ __forceinline__ int tile_split(int n_items, int most) {   // log2 of a tile's parts
+__device__ __forceinline__ int tile_split(int n_items, int most) {   // log2 of a tile's parts
     const int fits = n_items * 4 <= kGemmSlots ? 2 : (n_items * 2 <= kGemmSlots - kGemmSlots / 8 ? 1 : 0);
     return fits < most ? fits : most;
 }
